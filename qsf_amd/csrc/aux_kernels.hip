@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/qsf_types.h"
+#include "aux_device.hpp"
 #include "fft_core.hpp"
 #include "qsf_launch.hpp"
 
@@ -12,46 +13,10 @@ struct AxisTableBatch {
   AxisTableArgs a[24];
 };
 
-template <typename Real>
 __global__ void axis_tables_kernel(AxisTableBatch batch) {
-  using T = typename cvec<Real>::T;
   const AxisTableArgs& a = batch.a[blockIdx.y];
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
-  double h;
-  if (a.kind == 0) {  // X: potential (per-axis part) + x·F  (hamiltonian.h:44-79)
-    const double x = a.xmin + i * a.dx;
-    const double ne = a.use_ne ? a.NE / sqrt(x * x + a.Nsoft) : 0.0;
-    h = ne + x * a.C;
-  } else {            // P: ½p² + p·A
-    const double p = a.dp * (double)(i < a.pn2 ? i : i - a.pn);
-    h = (0.5 * p * p) + (p * a.C);
-  }
-  const double v = a.delta * h;
-  double re, im;
-  if (a.mode == QSF_MODE_IM) { re = exp(-v); im = 0.0; }
-  else { sincos(-v, &im, &re); }
-  if (a.kind == 0 && a.apply_abs && a.absorber != QSF_ABS_NONE) {
-    const int64_t half = a.n / 2;
-    const int64_t nd = i < half ? -i : i - a.n + 1;   // neg_dist_from_edge grid.h:181-185
-    const int64_t node = a.nCAP + nd;
-    if (node > 0) {
-      double f;
-      if (a.absorber == QSF_ABS_CAP) {
-        const double s4 = (double)(node * (node * (node * node)));
-        f = exp(-a.delta * s4 * a.eta);                  // absorbers.h:40-46, one axis
-      } else {
-        // cos(π/2 · node/nCAP) as the sine of the distance from the edge (never negative)
-        const double c = sin(0.5 * M_PI * (double)(a.nCAP - node) / (double)a.nCAP);
-        f = pow(pow(c, 0.125), a.delta / a.tau);         // cos^(1/8) per tau of time
-      }
-      re *= f;
-      im *= f;
-    }
-  }
-  re *= a.norm;
-  im *= a.norm;
-  reinterpret_cast<T*>(a.out)[i] = T{(Real)re, (Real)im};
+  if (i < a.n) reinterpret_cast<double2*>(a.out)[i] = axis_table_entry(a, i);
 }
 
 void launch_axis_tables(int precision, const AxisTableArgs* a, int count, hipStream_t s) {
@@ -67,7 +32,7 @@ void launch_axis_tables(int precision, const AxisTableArgs* a, int count, hipStr
     // phase tables are FP64 in both precisions: the FP32 step applies them with one FP64
     // product and a single rounding (a table rounded to FP32 once would bias every step)
     (void)precision;
-    hipLaunchKernelGGL(axis_tables_kernel<double>, grid, dim3(256), 0, s, b);
+    hipLaunchKernelGGL(axis_tables_kernel, grid, dim3(256), 0, s, b);
   }
 }
 

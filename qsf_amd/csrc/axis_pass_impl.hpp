@@ -46,6 +46,7 @@ template <typename T, bool WAVE = false> struct RowAddr {
   static constexpr int SH = sizeof(T) == 16 ? 4 : 5;
   static constexpr bool kWave = WAVE;
   static constexpr bool kSplitOk = false;
+  static constexpr bool kToggle = false;   // exchanges alternate between two LDS images
   int base;
   __device__ __forceinline__ int operator()(int p) const { return base + p + (p >> SH); }
 };
@@ -132,6 +133,7 @@ template <typename Real, int N, bool ROW, int V = 0> struct Geo {
 template <typename T, int W> struct ColAddr {
   static constexpr bool kWave = false;
   static constexpr bool kSplitOk = true;
+  static constexpr bool kToggle = false;
   int w;
   __device__ __forceinline__ int operator()(int p) const {
     const int a = p * W + w;

@@ -431,7 +431,8 @@ __device__ __forceinline__ void fft_stage(T* v, int t, T* lds, const Addr& addr,
     exchange_sync<Addr::kWave>();
 #pragma unroll
     for (int q = 0; q < E; ++q) v[q] = lds[addr(t + TT * q)];
-    exchange_sync<Addr::kWave>();
+    if constexpr (Addr::kToggle) addr.flip();   // the next exchange goes through the other image
+    else exchange_sync<Addr::kWave>();
   }
   if constexpr (!LAST && kSplitFor<T, Addr>) {
     // Exchange in two halves, real parts then imaginary parts: a block needs half the LDS, so

@@ -110,6 +110,58 @@ struct FluxArgs {
 };
 void launch_flux(const FluxArgs& a, hipStream_t s);
 
+// ---- lines: whole steps of a 1D propagation in one launch (line_impl.hpp) ----
+enum LineFlags : uint32_t {
+  LINE_OBS = 1u << 0,        // boundary observables of every step
+  LINE_EPOT = 1u << 1,
+  LINE_EKIN = 1u << 2,
+  LINE_FLUX = 1u << 3,       // gather the flux stencil of every step
+  LINE_NORMALIZE = 1u << 4,  // scale to unit norm at every boundary, before the observables
+  LINE_STOP = 1u << 5        // stop once the energy difference is within `accuracy`
+};
+struct LineParams {
+  void* psi;                 // in: step-boundary state, or (za_in) before its trailing X factor;
+                             // out: the latter, or with LINE_EKIN or LINE_NORMALIZE the former
+  const double2* za_in;      // trailing X factor of the step before the run, still to be applied
+  const void* roots;
+  int32_t steps, nsub;       // P substeps per step
+  uint32_t flags;
+  const double2* xtab;       // [step][nsub + 1][n] X factors, xtab_step elements per step (0: static)
+  const double2* ptab;       // [step][nsub][n] P factors
+  int64_t xtab_step, ptab_step;
+  const double* vtab;        // potential of the nodes
+  const double* kin_w;       // 1/2 p^2 of the nodes
+  const int32_t* gather_pos; // node of each flux stencil value
+  int32_t nvals;
+  void* gathered;            // [step][nvals]
+  double* sums;              // [step][wave][3]: norm, potential, kinetic
+  double dV, dVm, last_energy, accuracy;
+  int32_t* done;             // steps taken
+};
+// Launches the run; returns the waves per block (the layout of `sums`), also without launching
+// when p.psi is null; -1: unsupported length. `variant`: the tuned variant of the length's row pass.
+int launch_line(int precision, int64_t n, int variant, const LineParams& p, hipStream_t s);
+
+constexpr int kLineTables = 320, kLineSteps = 128;   // tables and steps of one run
+struct LineCouplings {
+  double C[kLineTables];
+  double delta[9];
+  int32_t per_step;          // tables per step
+};
+// `tables` tables of a.n entries at a.out, table k with coupling c.C[k] and substep length
+// c.delta[k % c.per_step].
+void launch_line_tables(const AxisTableArgs& a, const LineCouplings& c, int tables, hipStream_t s);
+void launch_line_potential(double* out, int64_t n, const ObsParams& o, hipStream_t s);
+struct LineRows {
+  const double* sums;
+  int32_t waves, nvals;
+  double* rec;               // [step][rec_width]: norm, epot, ekin, fluxes
+  int64_t rec_width;
+  FluxArgs flux;             // nb = 0: no fluxes
+};
+// c.C[s] is the velocity-gauge correction of step s's fluxes.
+void launch_line_rows(int precision, const LineRows& a, const LineCouplings& c, int steps, hipStream_t s);
+
 // Element-wise multiply of a complex (precision) array by a real FP64 table value per point.
 void launch_scale(int precision, void* psi, int64_t m, double s, hipStream_t st);
 void launch_copy_convert(int from_prec, const void* src, int to_prec, void* dst, int64_t m, hipStream_t s);

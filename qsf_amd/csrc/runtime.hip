@@ -189,6 +189,8 @@ struct Grid {
   std::vector<int> fftAxes;
   int pperm[3];
   DBuf psi, aux, partials, red, redscratch, kinw, masktab, invtab, corrtab, m1tab, tabs;
+  DBuf linetabs, linesums, linevals, linepot;   // workspaces of line runs (Prop::line_steps)
+  int linehalf = 0;
   std::map<int64_t, std::unique_ptr<DBuf>> roots;
   std::map<std::pair<int64_t, int>, std::unique_ptr<DBuf>> pairs;
   std::unique_ptr<Gather> gather;
@@ -383,6 +385,45 @@ struct Grid {
     return p;
   }
 
+  AxisTableArgs x_table_args(int a, int mode, double delta, double C, void* out) const {
+    AxisTableArgs t{};
+    t.out = out;
+    t.n = n[a];
+    t.kind = 0;
+    t.mode = mode;
+    t.delta = delta;
+    t.C = C;
+    t.xmin = xmin[a];
+    t.dx = dx[a];
+    t.use_ne = (d.potential != QSF_POT_NONE) && bounded[a] &&
+               (reduced() || (d.potential == QSF_POT_COULOMB && !radial));
+    t.NE = d.Ncharge * d.Echarge;
+    t.Nsoft = d.Nsoft;
+    t.absorber = d.absorber;
+    t.apply_abs = !many;
+    t.nCAP = d.nCAP;
+    t.eta = eta;
+    t.tau = d.absorber_tau;
+    t.norm = 1.0;
+    return t;
+  }
+  AxisTableArgs p_table_args(int a, int mode, double delta, double C, bool normalise, void* out) const {
+    AxisTableArgs t{};
+    const int sa = pperm[a];
+    t.out = out;
+    t.n = n[a];
+    t.kind = 1;
+    t.mode = mode;
+    t.delta = delta;
+    t.C = C;
+    t.dp = dp[sa];
+    t.pn = n[sa];
+    t.pn2 = n2[sa];
+    const bool fa = std::find(fftAxes.begin(), fftAxes.end(), a) != fftAxes.end();
+    t.norm = (normalise && fa) ? 1.0 / double(n[a]) : 1.0;
+    return t;
+  }
+
   // X factor of one X substep: per-axis tables built now + the static pair table.
   // X factors that do not couple (velocity gauge, no field term in X) depend on (mode, δ)
   // only: built once into tables of their own, so every step (and both X halves of a pass)
@@ -406,28 +447,7 @@ struct Grid {
       s = own->p;
     }
     AxisTableArgs args[3];
-    for (int a = 0; a < D; ++a) {
-      AxisTableArgs& t = args[a];
-      t = AxisTableArgs{};
-      t.out = slot_axis(s, a);
-      t.n = n[a];
-      t.kind = 0;
-      t.mode = mode;
-      t.delta = delta;
-      t.C = coupled ? C[a] : 0.0;
-      t.xmin = xmin[a];
-      t.dx = dx[a];
-      t.use_ne = (d.potential != QSF_POT_NONE) && bounded[a] &&
-                 (reduced() || (d.potential == QSF_POT_COULOMB && !radial));
-      t.NE = d.Ncharge * d.Echarge;
-      t.Nsoft = d.Nsoft;
-      t.absorber = d.absorber;
-      t.apply_abs = !many;
-      t.nCAP = d.nCAP;
-      t.eta = eta;
-      t.tau = d.absorber_tau;
-      t.norm = 1.0;
-    }
+    for (int a = 0; a < D; ++a) args[a] = x_table_args(a, mode, delta, coupled ? C[a] : 0.0, slot_axis(s, a));
     for (int a = 0; a < D; ++a) pending_tables.push_back(args[a]);
     XFactor f{};
     for (int a = 0; a < D; ++a) f.axis[a] = args[a].out;
@@ -462,22 +482,8 @@ struct Grid {
   void p_factor(int mode, double delta, const double* C, bool coupled, bool normalise, const void** pf) {
     void* s = next_slot();
     AxisTableArgs args[3];
-    for (int a = 0; a < D; ++a) {
-      AxisTableArgs& t = args[a];
-      t = AxisTableArgs{};
-      const int sa = pperm[a];
-      t.out = slot_axis(s, a);
-      t.n = n[a];
-      t.kind = 1;
-      t.mode = mode;
-      t.delta = delta;
-      t.C = coupled ? C[sa] : 0.0;
-      t.dp = dp[sa];
-      t.pn = n[sa];
-      t.pn2 = n2[sa];
-      const bool fa = std::find(fftAxes.begin(), fftAxes.end(), a) != fftAxes.end();
-      t.norm = (normalise && fa) ? 1.0 / double(n[a]) : 1.0;
-    }
+    for (int a = 0; a < D; ++a)
+      args[a] = p_table_args(a, mode, delta, coupled ? C[pperm[a]] : 0.0, normalise, slot_axis(s, a));
     for (int a = 0; a < D; ++a) pending_tables.push_back(args[a]);
     for (int a = 0; a < 3; ++a) pf[a] = a < D ? args[a].out : nullptr;
   }
@@ -875,6 +881,11 @@ struct Grid {
   }
 
   void flux_from_gather(const double* vgC, double* dev_out, double* accum, double w) {
+    FluxArgs f = flux_args(vgC, accum, w);
+    f.out = dev_out ? dev_out : gather->out.as<double>();
+    launch_flux(f, st());
+  }
+  FluxArgs flux_args(const double* vgC, double* accum, double w) const {
     FluxArgs f{};
     f.gathered = gather->values.p;
     f.precision = prec;
@@ -889,10 +900,9 @@ struct Grid {
     }
     f.scale = dV / dx[0];
     f.partials = gather->partials.as<double>();
-    f.out = dev_out ? dev_out : gather->out.as<double>();
     f.accum = accum;
     f.accum_weight = w;
-    launch_flux(f, st());
+    return f;
   }
 
   // flux of each border family into out (host); with accum, also accum[b] += flux * w on the
@@ -1175,11 +1185,15 @@ struct Prop {
   double dt, timer = 0, timer_copy = 0, state_accuracy = 0;
   double dif_energy = 1e300, last_change = 0;
   int exec = 0;
+  bool member_calls = false;   // qsf_prop_set_exec(1): one standalone call per reference member
+  bool line_open = false;      // line runs taken since the grid was last settled
+  DBuf linestatic;             // phase tables of a line run that do not change from step to step
   int width;
   // host rows; rows produced by fused passes are completed from the device on sync
   std::vector<double> rows;
   struct DevRow { int row; bool ekin; };
   std::vector<DevRow> pending_rows;
+  static constexpr int kRecWidth = 3 + 16;   // norm, epot, ekin, fluxes of a device row
   DBuf devrec, fluxint;
   int64_t devrec_cap = 0, devrec_used = 0;
   // fused pipeline state of each grid
@@ -1360,7 +1374,7 @@ struct Prop {
     }
   }
 
-  double* obs_row() { return devrec.as<double>() + (size_t)pend_row * (3 + 16); }
+  double* obs_row() { return devrec.as<double>() + (size_t)pend_row * kRecWidth; }
 
   void after_obs(Grid& g, int tiles) {
     // reduce [norm, epot] of the boundary state into this row's device record
@@ -1486,6 +1500,7 @@ struct Prop {
 
   // Apply whatever the pipeline left pending so every grid holds its step-boundary state.
   void flush() {
+    line_open = false;
     const bool post = pend_post;
     for (size_t r = 0; r < set->g.size(); ++r) {
       if (r == 1 && post) {
@@ -1560,7 +1575,7 @@ struct Prop {
     }
     if (!devrec.p) {
       devrec_cap = 4096;
-      devrec.ensure(devrec_cap * (3 + 16) * sizeof(double));
+      devrec.ensure(devrec_cap * kRecWidth * sizeof(double));
     }
     pend_obs = true;
     pend_row = (int)devrec_used++;
@@ -1572,18 +1587,24 @@ struct Prop {
   void sync_rows() {
     if (pending_rows.empty()) return;
     if (pend_obs) flush_obs_only();
-    std::vector<double> dev((size_t)devrec_used * (3 + 16));
+    std::vector<double> dev((size_t)devrec_used * kRecWidth);
     QSF_HIP(hipMemcpyAsync(dev.data(), devrec.p, dev.size() * sizeof(double), hipMemcpyDeviceToHost, st()));
     QSF_HIP(hipStreamSynchronize(st()));
     Grid& g = main();
     const int o = pd.outputs;
     for (size_t k = 0; k < pending_rows.size(); ++k) {
       double* row = &rows[(size_t)pending_rows[k].row * width];
-      const double* d = &dev[k * (3 + 16)];
+      const double* d = &dev[k * kRecWidth];
       if (o & QSF_OUT_NORM) row[2] = d[0] * g.dV;
       if (o & QSF_OUT_EPOT) row[3] = d[1] * g.dV;
       if (o & QSF_OUT_EKIN) row[4] = d[2] * g.dVm;
       if (o & QSF_OUT_ETOT) row[5] = d[1] * g.dV + d[2] * g.dVm;
+      if (o & QSF_OUT_EDIFF) {   // line runs only: the fused passes leave it to the member calls
+        const double curr = row[5] = d[1] * g.dV + d[2] * g.dVm;
+        dif_energy = row[6] = curr - last_change;
+        last_change = curr;
+        if (!(o & QSF_OUT_ETOT)) row[5] = std::nan("");
+      }
       if (o & QSF_OUT_FLUX)
         for (int b = 0; b < pd.nborders; ++b) row[7 + b] = d[3 + b];
     }
@@ -1593,9 +1614,178 @@ struct Prop {
 
   void flush_obs_only() { flush(); }
 
-  // the fused pipeline left work for the next pass (the grids are not at the step boundary)
+  // ---- lines: runs of whole steps in one launch (line_impl.hpp) ----
+  // Every 1D propagation, unless its member calls were asked for; a steering energy difference
+  // needs both energies on the device.
+  bool line_path() const {
+    if (!set || member_calls || set->g.size() != 1 || set->D != 1) return false;
+    const int both = QSF_OUT_EPOT | QSF_OUT_EKIN;
+    return exec == 0 || !(pd.outputs & (QSF_OUT_ETOT | QSF_OUT_EDIFF)) || (pd.outputs & both) == both;
+  }
+
+  // At most `want` steps, as many as one run holds; returns the steps taken (fewer only where the
+  // energy difference stopped the run).
+  int64_t line_steps(int64_t want) {
+    Grid& g = main();
+    const int K = (int)chains.size(), N = (int)g.n[0];
+    const bool cx = couples() == QSF_REP_X;
+    const int per = cx ? K + 1 : K, still = cx ? K : K + 1;
+    const int o = pd.outputs;
+    int64_t run = std::min<int64_t>(want, std::min(kLineSteps, kLineTables / per));
+    if (o) {
+      if (!devrec.p) {
+        devrec_cap = 4096;
+        devrec.ensure(devrec_cap * kRecWidth * sizeof(double));
+      }
+      if (devrec_used >= devrec_cap) sync_rows();
+      run = std::min(run, devrec_cap - devrec_used);
+    }
+    // host side of the steps: couplings, times and rows
+    const phys::Coupling coup0 = coup;
+    const double timer0 = timer;
+    const int64_t step0 = step;
+    const size_t rows0 = rows.size(), pending0 = pending_rows.size();
+    const bool ekin = o & (QSF_OUT_EKIN | QSF_OUT_ETOT);
+    LineCouplings moving{}, fixed{}, after{};
+    moving.per_step = per;
+    fixed.per_step = still;
+    for (int64_t s = 0; s < run; ++s) {
+      const auto ops = schedule();
+      int im = 0, is = 0;
+      for (const SubOp& op : ops) {
+        if ((op.rep == QSF_REP_X) == cx) {
+          moving.delta[im] = op.delta;
+          moving.C[s * per + im++] = op.C[0];
+        } else {
+          fixed.delta[is++] = op.delta;
+        }
+      }
+      double c3[3];
+      coup.values(c3);
+      after.C[s] = cx ? 0.0 : c3[0];
+      if (o) {
+        std::vector<double> row(width, std::nan(""));
+        row[0] = (double)step;
+        row[1] = timer;
+        pending_rows.push_back({(int)(rows.size() / width), ekin});
+        rows.insert(rows.end(), row.begin(), row.end());
+      }
+    }
+    // two buffers in turn: the run before may have left its last table pending
+    g.linetabs.ensure((size_t)2 * kLineTables * N * Grid::kTabBytes);
+    g.linehalf ^= 1;
+    double2* mt = g.linetabs.as<double2>() + (size_t)g.linehalf * kLineTables * N;
+    auto args = [&](bool x, void* out) {
+      return x ? g.x_table_args(0, pd.mode, 0.0, 0.0, out) : g.p_table_args(0, pd.mode, 0.0, 0.0, true, out);
+    };
+    if (!linestatic.p) {
+      linestatic.ensure((size_t)still * N * Grid::kTabBytes);
+      launch_line_tables(args(!cx, linestatic.p), fixed, still, st());
+    }
+    launch_line_tables(args(cx, mt), moving, (int)run * per, st());
+    if (!g.linepot.p) {
+      ObsParams ob{};
+      g.obs_params(ob, true);
+      g.linepot.ensure(N * sizeof(double));
+      launch_line_potential(g.linepot.as<double>(), N, ob, st());
+    }
+    LineParams p{};
+    const int var = ctx->variant_of(g.prec, 1, N, g.m);
+    const int waves = launch_line(g.prec, N, var, p, st());
+    QSF_REQUIRE(waves > 0, QSF_ERR_UNSUPPORTED, "no FFT kernel for this axis length");
+    g.linesums.ensure(((size_t)kLineSteps * waves * 3 + 1) * sizeof(double));
+    p.psi = g.psi.p;
+    p.roots = g.root(N);
+    p.steps = (int)run;
+    p.nsub = K;
+    const double2* ft = linestatic.as<double2>();
+    p.xtab = cx ? mt : ft;
+    p.xtab_step = cx ? (int64_t)per * N : 0;
+    p.ptab = cx ? ft : mt;
+    p.ptab_step = cx ? 0 : (int64_t)per * N;
+    if (deferred[0] && pend[0].on) p.za_in = static_cast<const double2*>(pend[0].f.axis[0]);
+    p.vtab = g.linepot.as<double>();
+    p.kin_w = g.kinw.as<double>();
+    p.dV = g.dV;
+    p.dVm = g.dVm;
+    p.sums = g.linesums.as<double>();
+    p.done = reinterpret_cast<int32_t*>(p.sums + (size_t)kLineSteps * waves * 3);
+    const bool flux = (o & QSF_OUT_FLUX) && pd.nborders > 0;
+    const bool steers = pd.mode == QSF_MODE_IM && (o & QSF_OUT_EDIFF);
+    if (o) p.flags |= LINE_OBS;
+    if (o & QSF_OUT_EPOT) p.flags |= LINE_EPOT;
+    if (ekin) p.flags |= LINE_EKIN;
+    if (o & QSF_OUT_NORMALIZE) p.flags |= LINE_NORMALIZE;
+    if (flux) {
+      g.build_gather(pd.borders, pd.nborders);
+      p.flags |= LINE_FLUX;
+      p.gather_pos = g.gather->pos.as<int32_t>();
+      p.nvals = (int32_t)g.gather->nvals;
+      // the arithmetic's complex type, 16 bytes at most
+      g.linevals.ensure((size_t)kLineSteps * std::max<int64_t>(g.gather->nvals, 1) * 16);
+      p.gathered = g.linevals.p;
+    }
+    if (steers) {
+      p.flags |= LINE_STOP;
+      p.last_energy = last_change;
+      p.accuracy = state_accuracy;
+    }
+    hipEvent_t ea = nullptr, eb = nullptr;
+    if (ctx->prof) {
+      ea = ctx->event();
+      eb = ctx->event();
+      QSF_HIP(hipEventRecord(ea, st()));
+    }
+    launch_line(g.prec, N, var, p, st());
+    QSF_HIP(hipGetLastError());
+    if (ctx->prof) {
+      QSF_HIP(hipEventRecord(eb, st()));
+      const char* pr = g.prec == QSF_FP64 ? "f64" : (g.prec == QSF_FP32_STATE ? "s32" : "f32");
+      ctx->launches.push_back({std::string("line_") + pr + "_n" + std::to_string(N), ea, eb, 2.0 * N * g.cb});
+      if (ctx->launches.size() >= 4096) drain_prof(ctx);
+    }
+    int32_t done = (int32_t)run;
+    if (steers) {
+      QSF_HIP(hipMemcpyAsync(&done, p.done, sizeof(done), hipMemcpyDeviceToHost, st()));
+      QSF_HIP(hipStreamSynchronize(st()));
+    }
+    if (o && done > 0) {
+      LineRows r{};
+      r.sums = p.sums;
+      r.waves = waves;
+      r.nvals = p.nvals;
+      r.rec = devrec.as<double>() + (size_t)devrec_used * kRecWidth;
+      r.rec_width = kRecWidth;
+      if (flux) {
+        r.flux = g.flux_args(nullptr, fluxint.as<double>(), dt);
+        r.flux.gathered = p.gathered;
+      }
+      launch_line_rows(g.prec, r, after, done, st());
+      QSF_HIP(hipGetLastError());
+      devrec_used += done;
+    }
+    if (done < run) {
+      // the run stopped early: the host side goes back to the steps that were taken
+      coup = coup0;
+      timer = timer0;
+      step = step0;
+      for (int32_t s = 0; s < done; ++s) schedule();
+      rows.resize(rows0 + (size_t)done * width);
+      pending_rows.resize(pending0 + done);
+    }
+    deferred[0] = pend[0].on = !(o && (ekin || (o & QSF_OUT_NORMALIZE)));
+    pend[0].f = XFactor{};
+    pend[0].f.axis[0] = p.xtab + (run - 1) * p.xtab_step + (int64_t)K * N;
+    line_open = true;
+    if (steers) sync_rows();   // the energy difference the loop is steered by
+    return done;
+  }
+
+  // the fused pipeline left work for the next pass (the grids are not at the step boundary), or
+  // line runs since the last settle (their grid is at the boundary, and settling costs nothing)
   bool pending() const {
     if (!fused()) return false;
+    if (line_open) return true;
     for (size_t r = 0; r < deferred.size(); ++r)
       if (deferred[r] || pend[r].on) return true;
     return pend_obs || pend_post;
@@ -1643,8 +1833,17 @@ struct Prop {
     if (pd.mode == QSF_MODE_RE) return step <= max_steps;
     return std::fabs(dif_energy) > state_accuracy && step != max_steps;
   }
+  // steps the loop would still take if no energy difference ended it
+  int64_t steps_left() const {
+    if (pd.mode == QSF_MODE_RE) return max_steps - step + 1;
+    return step < max_steps ? max_steps - step : INT64_MAX;   // `step != max_steps` never ends past it
+  }
   void start() { compute_each(); }
   void loop_body() {
+    if (line_path()) {
+      line_steps(1);
+      return;
+    }
     make_step();
     compute_each();
     post_compute();
@@ -2405,8 +2604,12 @@ int qsf_prop_run_steps(qsf_prop* p, int64_t k, int64_t* done) {
     require_set(p);
     int64_t i = 0;
     while (i < k && p->p.should_continue()) {
-      p->p.loop_body();
-      ++i;
+      if (p->p.line_path()) {
+        i += p->p.line_steps(std::min(k - i, p->p.steps_left()));
+      } else {
+        p->p.loop_body();
+        ++i;
+      }
     }
     if (done) *done = i;
   });
@@ -2551,7 +2754,9 @@ int qsf_prop_set_exec(qsf_prop* p, int mode) {
     QSF_REQUIRE(mode == 1 || !(p->p.set->multi && p->p.set->D == 3), QSF_ERR_UNSUPPORTED,
                 "3D multigrid sets run unfused");
     p->p.flush();
+    p->p.sync_rows();   // rows of line runs come before the member calls' rows
     p->p.exec = mode;
+    p->p.member_calls = mode == 1;
   });
 }
 
