@@ -84,8 +84,8 @@ __global__ void line_rows_kernel(LineRows a, LineCouplings c) {
   }
 }
 
-// The flux time integrals take the run's rows in step order, whatever runs the steps came in.
-__global__ void line_integral_kernel(LineRows a, int steps) {
+// The flux time integrals take a run's rows in step order, whatever runs the steps came in.
+__global__ void row_integral_kernel(LineRows a, int steps) {
   const int b = threadIdx.x;
   if (b >= a.flux.nb) return;
   double x = a.flux.accum[b];
@@ -94,13 +94,16 @@ __global__ void line_integral_kernel(LineRows a, int steps) {
   a.flux.accum[b] = x;
 }
 
+void launch_row_integral(const LineRows& a, int steps, hipStream_t s) {
+  hipLaunchKernelGGL(row_integral_kernel, dim3(1), dim3(64), 0, s, a, steps);
+}
+
 void launch_line_rows(int precision, const LineRows& a, const LineCouplings& c, int steps, hipStream_t s) {
   if (precision == QSF_FP32_MIXED)
     hipLaunchKernelGGL(line_rows_kernel<float>, dim3((unsigned)steps), dim3(64), 0, s, a, c);
   else
     hipLaunchKernelGGL(line_rows_kernel<double>, dim3((unsigned)steps), dim3(64), 0, s, a, c);
-  if (a.flux.nb > 0 && a.flux.accum)
-    hipLaunchKernelGGL(line_integral_kernel, dim3(1), dim3(64), 0, s, a, steps);
+  if (a.flux.nb > 0 && a.flux.accum) launch_row_integral(a, steps, s);
 }
 
 }  // namespace qsf

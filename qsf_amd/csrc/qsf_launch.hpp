@@ -161,6 +161,8 @@ struct LineRows {
 };
 // c.C[s] is the velocity-gauge correction of step s's fluxes.
 void launch_line_rows(int precision, const LineRows& a, const LineCouplings& c, int steps, hipStream_t s);
+// The flux time integrals of `steps` rows, added in step order.
+void launch_row_integral(const LineRows& a, int steps, hipStream_t s);
 
 // Element-wise multiply of a complex (precision) array by a real FP64 table value per point.
 void launch_scale(int precision, void* psi, int64_t m, double s, hipStream_t st);

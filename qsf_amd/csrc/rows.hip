@@ -1,0 +1,141 @@
+// rows.hip — record rows of several step boundaries reduced together. A boundary's sums and fluxes
+// are small work (a few blocks, each with barriers between its levels): one at a time they cost
+// 23 us of a 44 us step of a 256^2 plane (reduction 3.8, flux 9.5, its second level 9.6), and for
+// up to kRowSlots boundaries together about the same once. The sums and their order are those of the
+// single-boundary kernels, so the rows have the same bits.
+#include <hip/hip_runtime.h>
+
+#include "../../include/qsf_types.h"
+#include "fft_core.hpp"
+#include "rows.hpp"
+
+namespace qsf {
+
+// Norm and potential sums of slot blockIdx.y: block x takes chunk x of the slot's tiles (one chunk
+// of all tiles where they are few).
+__global__ void rows_reduce_kernel(const double* in, int64_t slot_stride, int64_t count, int width, int64_t chunk,
+                                   double* out, int64_t out_stride) {
+  __shared__ double red[256];
+  const double* p = in + (int64_t)blockIdx.y * slot_stride;
+  const int64_t lo = (int64_t)blockIdx.x * chunk, hi = lo + chunk < count ? lo + chunk : count;
+  for (int c = 0; c < 2; ++c) {
+    double acc = 0.0;
+    for (int64_t k = lo + threadIdx.x; k < hi; k += 256) acc += p[k * width + c];
+    red[threadIdx.x] = acc;
+    block_sync();
+    for (int s = 128; s > 0; s >>= 1) {
+      if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+      block_sync();
+    }
+    if (threadIdx.x == 0) out[(int64_t)blockIdx.y * out_stride + blockIdx.x * 2 + c] = red[0];
+    block_sync();
+  }
+}
+
+template <typename Real, int D>
+__global__ void rows_flux_kernel(RowSlots r) {
+  using T = typename cvec<Real>::T;
+  const FluxArgs& a = r.flux;
+  const T* g = reinterpret_cast<const T*>(a.gathered) + (int64_t)blockIdx.y * r.nvals;
+  const double* C = r.C[blockIdx.y];
+  const int nb = a.nb;
+  constexpr int stride = 1 + 2 * D;
+  double acc[16];
+#pragma unroll
+  for (int b = 0; b < 16; ++b) acc[b] = 0.0;
+  for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < a.npts;
+       p += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t* q = a.pts + p * stride;
+    const T c = g[q[0]];
+    const double cr = c.x, ci = c.y, nrm = cr * cr + ci * ci;
+    double j[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      j[d] = 0.0;
+      const int32_t sp = q[1 + d], sm = q[1 + D + d];
+      if (sp >= 0 && sm >= 0) {
+        // inv_2dx * Im(conj(ψ_c) (ψ_+ - ψ_-))  (grid.h:467-481)
+        const double dr = (double)g[sp].x - (double)g[sm].x, di = (double)g[sp].y - (double)g[sm].y;
+        j[d] = a.inv_2dx[d] * (cr * di - ci * dr);
+      }
+      j[d] += C[d] * nrm;  // velocityGaugeCorrection (propagator.h:249-257)
+    }
+    const double* bv = a.bvec + p * nb * D;
+#pragma unroll
+    for (int b = 0; b < 16; ++b) {
+      if (b >= nb) break;
+      double s = 0.0;
+#pragma unroll
+      for (int d = 0; d < D; ++d) s += j[d] * bv[b * D + d];
+      acc[b] += s;
+    }
+  }
+  __shared__ double red[256];
+#pragma unroll
+  for (int b = 0; b < 16; ++b) {
+    if (b >= nb) break;
+    red[threadIdx.x] = acc[b];
+    block_sync();
+    for (int s = 128; s > 0; s >>= 1) {
+      if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+      block_sync();
+    }
+    if (threadIdx.x == 0) a.partials[((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * nb + b] = red[0];
+    block_sync();
+  }
+}
+
+// One block per slot and border: the fixed tree of flux_finish_kernel over the flux blocks.
+__global__ void rows_flux_finish_kernel(RowSlots r, int blocks) {
+  __shared__ double red[256];
+  const int b = blockIdx.x, nb = r.flux.nb;
+  const double* p = r.flux.partials + (int64_t)blockIdx.y * blocks * nb;
+  double acc = 0.0;
+  for (int64_t k = threadIdx.x; k < blocks; k += blockDim.x) acc += p[k * nb + b];
+  red[threadIdx.x] = acc;
+  block_sync();
+  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
+    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+    block_sync();
+  }
+  if (threadIdx.x == 0) r.rec[(int64_t)blockIdx.y * r.rec_width + 3 + b] = red[0] * r.flux.scale;
+}
+
+int flux_blocks(int64_t npts) {
+  const int64_t want = (npts + 255) / 256;
+  return (int)(want < 1 ? 1 : (want > 1024 ? 1024 : want));
+}
+
+void launch_rows(int precision, const RowSlots& a, int slots, hipStream_t s) {
+  if (a.tiles <= 4096) {
+    hipLaunchKernelGGL(rows_reduce_kernel, dim3(1, (unsigned)slots), dim3(256), 0, s, a.partials, a.tiles * 3, a.tiles, 3,
+                       a.tiles, a.rec, a.rec_width);
+  } else {
+    const int64_t chunk = (a.tiles + 255) / 256;
+    hipLaunchKernelGGL(rows_reduce_kernel, dim3(256, (unsigned)slots), dim3(256), 0, s, a.partials, a.tiles * 3, a.tiles,
+                       3, chunk, a.scratch, (int64_t)512);
+    hipLaunchKernelGGL(rows_reduce_kernel, dim3(1, (unsigned)slots), dim3(256), 0, s, (const double*)a.scratch,
+                       (int64_t)512, (int64_t)256, 2, (int64_t)256, a.rec, a.rec_width);
+  }
+  if (a.flux.nb <= 0) return;
+  const int blocks = flux_blocks(a.flux.npts);
+  const dim3 grid((unsigned)blocks, (unsigned)slots);
+  const bool f64 = precision == QSF_FP64;
+  if (a.flux.D == 2) {
+    if (f64) hipLaunchKernelGGL((rows_flux_kernel<double, 2>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((rows_flux_kernel<float, 2>), grid, dim3(256), 0, s, a);
+  } else {
+    if (f64) hipLaunchKernelGGL((rows_flux_kernel<double, 3>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((rows_flux_kernel<float, 3>), grid, dim3(256), 0, s, a);
+  }
+  hipLaunchKernelGGL(rows_flux_finish_kernel, dim3((unsigned)a.flux.nb, (unsigned)slots), dim3(256), 0, s, a, blocks);
+  if (a.flux.accum) {
+    LineRows l{};
+    l.rec = a.rec;
+    l.rec_width = a.rec_width;
+    l.flux = a.flux;
+    launch_row_integral(l, slots, s);
+  }
+}
+
+}  // namespace qsf

@@ -1,0 +1,23 @@
+#pragma once
+// rows.hpp — record rows of several step boundaries reduced together (rows.hip).
+#include <hip/hip_runtime.h>
+
+#include "qsf_launch.hpp"
+
+namespace qsf {
+
+constexpr int kRowSlots = 32;   // boundaries one reduction takes
+struct RowSlots {
+  const double* partials;    // [slot][tiles][3] block sums of the observing passes
+  int64_t tiles;
+  double* rec;               // [slot][rec_width]: norm and potential sums, kinetic (not written), fluxes
+  int64_t rec_width;
+  double* scratch;           // [slot][256 * 2] second reduction level (more than 4096 tiles)
+  FluxArgs flux;             // nb = 0: no fluxes; gathered: [slot][nvals]; partials: [slot][blocks * nb]
+  int64_t nvals;
+  double C[kRowSlots][3];    // velocity-gauge correction of each boundary
+};
+int flux_blocks(int64_t npts);
+void launch_rows(int precision, const RowSlots& a, int slots, hipStream_t s);
+
+}  // namespace qsf

@@ -22,6 +22,7 @@
 #include "../../include/qsf_hip.h"
 #include "physics.hpp"
 #include "qsf_launch.hpp"
+#include "rows.hpp"
 
 namespace qsf {
 
@@ -521,16 +522,14 @@ struct Grid {
     pending_tables.clear();
   }
 
-  // `single_out`: where the three block sums go when the pass is one tile (they are then the
-  // final sums and need no reduction launch)
-  int run(PassParams& p, int force_variant = -1, double* single_out = nullptr) {
+  int variant(const PassParams& p) const { return ctx->variant_of(prec, tune_class(p), n[p.axis], m); }
+
+  int run(PassParams& p, int force_variant = -1) {
     build_tables();
-    const int var = force_variant >= 0 ? force_variant : ctx->variant_of(prec, tune_class(p), n[p.axis], m);
-    if (p.flags & F_OBS) {
-      int64_t tiles = axis_pass_tiles(prec, p, var);
-      partials.ensure(tiles * 3 * sizeof(double));
-      if (tiles == 1 && single_out) p.obs.partials = single_out;
-      if (!p.obs.partials) p.obs.partials = partials.as<double>();
+    const int var = force_variant >= 0 ? force_variant : variant(p);
+    if ((p.flags & F_OBS) && !p.obs.partials) {
+      partials.ensure(axis_pass_tiles(prec, p, var) * 3 * sizeof(double));
+      p.obs.partials = partials.as<double>();
     }
     hipEvent_t ea = nullptr, eb = nullptr;
     if (ctx->prof) {
@@ -860,10 +859,10 @@ struct Grid {
   // The stencil values of the X state ahead of the pass that observes it, with the pending X
   // factor (or none) applied at each point: what that pass would gather, read from HBM instead
   // of from the pass's registers (for passes whose input is the X state).
-  void gather_ahead(const XFactor* xa) {
+  void gather_ahead(const XFactor* xa, void* out) {
     GatherXArgs a{};
     a.psi = psi.p;
-    a.out = gather->values.p;
+    a.out = out;
     a.row = gather->rowidx.as<int32_t>();
     a.pos = gather->pos.as<int32_t>();
     a.nvals = gather->nvals;
@@ -1307,13 +1306,28 @@ struct Prop {
     pend_post = false;
   }
 
-  void exec_fused(const std::vector<SubOp>& ops) {
-    // every phase table of this step first (each grid's own ring of slots), so the tables of
-    // all region grids build in one batched launch instead of one launch per pass
-    struct Sub { XFactor fb; const void* pf[3]; };
+  // One step as the host sees it: its substeps and phase tables, and the clock after it.
+  struct Sub { XFactor fb; const void* pf[3]; };
+  struct Plan {
+    std::vector<SubOp> ops;
+    std::vector<std::vector<Sub>> subs;   // per region grid, one per P substep
+    std::vector<XFactor> last;            // per region grid: the trailing X factor
+    int64_t step;
+    double timer, C[3];
+  };
+
+  // Advances the host side by one step; the tables it asks for (each grid's own ring of slots) are
+  // built by the set's next build_tables.
+  Plan plan_step() {
+    Plan q;
+    q.ops = schedule();
+    q.step = step;
+    q.timer = timer;
+    coup.values(q.C);
+    const auto& ops = q.ops;
     const size_t R = set->g.size();
-    std::vector<std::vector<Sub>> subs(R);
-    std::vector<XFactor> last(R);
+    q.subs.resize(R);
+    q.last.resize(R);
     for (size_t r = 0; r < R; ++r) {
       Grid& g = *set->g[r];
       for (size_t SI = 0; SI < ops.size(); ++SI) {
@@ -1323,12 +1337,41 @@ struct Prop {
         Sub sb;
         sb.fb = g.x_factor(pd.mode, xb.delta, xb.C, couples() == QSF_REP_X);
         g.p_factor(pd.mode, o.delta, o.C, couples() == QSF_REP_P, true, sb.pf);
-        subs[r].push_back(sb);
+        q.subs[r].push_back(sb);
       }
       const SubOp& xl = ops.back();
-      last[r] = g.x_factor(pd.mode, xl.delta, xl.C, couples() == QSF_REP_X);
+      q.last[r] = g.x_factor(pd.mode, xl.delta, xl.C, couples() == QSF_REP_X);
     }
-    set->build_tables();
+    return q;
+  }
+
+  // Steps whose tables are built by one launch: as many as the ring of slots holds beside the
+  // pending factor of the step before them.
+  int64_t plan_ahead() const {
+    const int K = (int)chains.size();
+    const int per = couples() == QSF_REP_X ? 2 * K + 1 : K;
+    return std::max(1, std::min(16, (Grid::kSlots - 2) / per - 1));
+  }
+
+  void run_fused(int64_t steps) {
+    while (steps > 0) {
+      const int64_t n = std::min(steps, plan_ahead());
+      std::vector<Plan> plans;
+      for (int64_t k = 0; k < n; ++k) plans.push_back(plan_step());
+      set->build_tables();
+      for (const Plan& q : plans) {
+        exec_fused(q);
+        if (pd.outputs) request_row(q);
+        post_compute();
+      }
+      steps -= n;
+    }
+    drain_rows();   // nothing waits in a slot between calls
+  }
+
+  void exec_fused(const Plan& plan) {
+    const std::vector<SubOp>& ops = plan.ops;
+    const size_t R = set->g.size();
     for (size_t r = 0; r < R; ++r) {
       Grid& g = *set->g[r];
       if (r == 1 && pend_post) run_receives();
@@ -1337,11 +1380,11 @@ struct Prop {
       for (size_t SI = 0; SI < ops.size(); ++SI) {
         if (ops[SI].rep != QSF_REP_P) continue;
         const bool first = (SI == 1);
-        const Sub& sb = subs[r][k++];
+        const Sub& sb = plan.subs[r][k++];
         run_p_substep(g, r, sb.fb, sb.pf, first && obs_here, first && r == 0 && pend_post);
       }
       pend[r].on = true;
-      pend[r].f = last[r];
+      pend[r].f = plan.last[r];
       deferred[r] = true;
     }
     if (pend_obs) pend_obs = false;
@@ -1364,10 +1407,72 @@ struct Prop {
     g.fill_mask(p);
   }
 
+  // ---- boundary observations: sums and flux stencils wait in slots and are reduced together ----
+  bool fluxes() const { return pd.nborders > 0 && (pd.outputs & QSF_OUT_FLUX); }
+  int64_t slot_tiles = 0, slot_vals = 0;
+  int slot_cap = 0, slots = 0, slot_row = 0;   // slot k holds the boundary of record row slot_row + k
+  double slot_C[kRowSlots][3];
+  DBuf slot_partials, slot_values, slot_scratch, slot_flux;
+
+  void ensure_slots(Grid& g, int64_t tiles) {
+    const int64_t vals = fluxes() ? g.gather->nvals : 0;
+    if (slot_cap && tiles == slot_tiles && vals == slot_vals) return;
+    drain_rows();
+    slot_tiles = tiles;
+    slot_vals = vals;
+    // 64 MiB of slots: all of them for planes, one or two for the largest cubes, whose single
+    // boundary is work enough for the device
+    const int64_t bytes = tiles * 3 * (int64_t)sizeof(double) + vals * (int64_t)g.cb;
+    slot_cap = (int)std::max<int64_t>(1, std::min<int64_t>(kRowSlots, (int64_t(64) << 20) / std::max<int64_t>(bytes, 1)));
+    slot_partials.ensure((size_t)slot_cap * tiles * 3 * sizeof(double));
+    slot_values.ensure((size_t)slot_cap * std::max<int64_t>(vals, 1) * g.cb);
+    slot_scratch.ensure((size_t)slot_cap * 512 * sizeof(double));
+    if (fluxes()) slot_flux.ensure((size_t)slot_cap * flux_blocks(g.gather->npts) * pd.nborders * sizeof(double));
+  }
+
+  void drain_rows() {
+    if (!slots) return;
+    Grid& g = main();
+    double* rec = devrec.as<double>() + (size_t)slot_row * kRecWidth;
+    if (slots == 1) {   // one boundary: the single-row kernels, which finish its fluxes in fewer launches
+      launch_reduce_partials(slot_partials.as<double>(), slot_tiles, 3, rec, slot_scratch.as<double>(), st(), 2);
+      if (fluxes()) {
+        FluxArgs f = g.flux_args(slot_C[0], fluxint.as<double>(), dt);
+        f.gathered = slot_values.p;
+        f.out = rec + 3;
+        launch_flux(f, st());
+      }
+    } else {
+      RowSlots r{};
+      r.partials = slot_partials.as<double>();
+      r.tiles = slot_tiles;
+      r.rec = rec;
+      r.rec_width = kRecWidth;
+      r.scratch = slot_scratch.as<double>();
+      r.nvals = slot_vals;
+      if (fluxes()) {
+        r.flux = g.flux_args(nullptr, fluxint.as<double>(), dt);
+        r.flux.gathered = slot_values.p;
+        r.flux.partials = slot_flux.as<double>();
+      }
+      std::memcpy(r.C, slot_C, sizeof(slot_C));
+      launch_rows(g.prec, r, slots, st());
+    }
+    QSF_HIP(hipGetLastError());
+    slots = 0;
+  }
+
   void obs_into(Grid& g, PassParams& p) {
     p.flags |= F_OBS;
     g.obs_params(p.obs, (pd.outputs & QSF_OUT_EPOT) != 0);
-    if (pd.nborders > 0 && (pd.outputs & QSF_OUT_FLUX)) g.set_gather(p.obs);
+    const int64_t tiles = axis_pass_tiles(g.prec, p, g.variant(p));
+    ensure_slots(g, tiles);
+    if (slots == slot_cap || (slots && pend_row != slot_row + slots)) drain_rows();
+    p.obs.partials = slot_partials.as<double>() + (size_t)slots * tiles * 3;
+    if (fluxes()) {
+      g.set_gather(p.obs);
+      p.obs.gather_out = slot_values.as<char>() + (size_t)slots * slot_vals * g.cb;
+    }
     if (pend_ekin) {
       g.aux.ensure(g.m * g.cb);
       p.obs.copy_out = g.aux.p;
@@ -1376,12 +1481,12 @@ struct Prop {
 
   double* obs_row() { return devrec.as<double>() + (size_t)pend_row * kRecWidth; }
 
-  void after_obs(Grid& g, int tiles) {
-    // reduce [norm, epot] of the boundary state into this row's device record
+  void after_obs(Grid& g) {
+    // the boundary's sums and stencil stay in their slot until drain_rows
+    if (!slots) slot_row = pend_row;
+    for (int a = 0; a < 3; ++a) slot_C[slots][a] = couples() == QSF_REP_P ? pend_obs_C[a] : 0.0;
+    ++slots;
     double* rec = obs_row();
-    if (tiles > 1) launch_reduce_partials(g.partials.as<double>(), tiles, 3, rec, g.redscratch.as<double>(), st());
-    if (pd.nborders > 0 && (pd.outputs & QSF_OUT_FLUX))
-      g.flux_from_gather(couples() == QSF_REP_P ? pend_obs_C : nullptr, rec + 3, fluxint.as<double>(), dt);
     if (pend_ekin) {
       // kinetic energy: forward transform of the copied boundary state, then <½p²>
       Grid& gg = g;
@@ -1422,10 +1527,9 @@ struct Prop {
       p.xb = fb;
       if (defer && pend[r].on) { p.flags |= F_XA; p.xa = pend[r].f; }
       for (int a = 0; a < 3; ++a) p.pf[a] = pf[a];
-      int tiles = 0;
       if (observe) obs_into(g, p);
-      tiles = g.run(p, -1, observe ? obs_row() : nullptr);
-      if (observe) after_obs(g, tiles);
+      g.run(p);
+      if (observe) after_obs(g);
       deferred[r] = true;
       pend[r].on = false;
       return;
@@ -1448,14 +1552,14 @@ struct Prop {
             if (p.obs.gather_rowptr) {
               // the state is in X before this pass: its flux stencil is read ahead, so the pass
               // does no gather (a row pass's gather costs it more than this read)
-              g.gather_ahead(pend[r].on ? &pend[r].f : nullptr);
+              g.gather_ahead(pend[r].on ? &pend[r].f : nullptr, p.obs.gather_out);
               p.obs.gather_rowptr = nullptr;
               p.obs.gather_pos = nullptr;
               p.obs.gather_out = nullptr;
             }
           }
-          int tiles = g.run(p, -1, observe ? obs_row() : nullptr);
-          if (observe) after_obs(g, tiles);
+          g.run(p);
+          if (observe) after_obs(g);
         } else {
           g.run(p);
         }
@@ -1475,8 +1579,8 @@ struct Prop {
         if (post) add_post(g, p);
       }
       if (observe) obs_into(g, p);
-      int tiles = g.run(p, -1, observe ? obs_row() : nullptr);
-      if (observe) after_obs(g, tiles);
+      g.run(p);
+      if (observe) after_obs(g);
     }
     for (int a = D - 2; a >= 1; --a) {  // middle axes forward
       PassParams p = g.params(a, g.psi.p, g.psi.p);
@@ -1518,55 +1622,63 @@ struct Prop {
       if (r == 0 && post) add_post(g, p);
       if (observe) obs_into(g, p);
       if (p.flags) {
-        int tiles = g.run(p, -1, observe ? obs_row() : nullptr);
-        if (observe) after_obs(g, tiles);
+        g.run(p);
+        if (observe) after_obs(g);
       }
       deferred[r] = false;
       pend[r].on = false;
     }
     pend_obs = false;
     pend_post = false;
+    drain_rows();
   }
 
   // ---- computeEach (propagator.h:275-300), canonical output order of qsf_types.h ----
-  void request_row(bool fused) {
+  std::vector<double> empty_row(int64_t at_step, double at_time) const {
+    std::vector<double> row(width, std::nan(""));
+    row[0] = (double)at_step;
+    row[1] = at_time;
+    return row;
+  }
+
+  // the row of the present boundary, by member calls
+  void request_row() {
     const double nan = std::nan("");
-    std::vector<double> row(width, nan);
-    row[0] = (double)step;
-    row[1] = timer;
+    std::vector<double> row = empty_row(step, timer);
     const int o = pd.outputs;
-    if (!fused) {
-      Grid& g = main();
-      if (o & QSF_OUT_NORMALIZE) g.normalize();
-      double r3[3] = {nan, nan, nan};
-      if (o & (QSF_OUT_NORM | QSF_OUT_EPOT)) g.observe((o & QSF_OUT_EPOT) != 0, false, r3);
-      if (o & QSF_OUT_NORM) row[2] = r3[0] * g.dV;
-      double epot = nan, ekin = nan;
-      if (o & QSF_OUT_EPOT) row[3] = epot = r3[1] * g.dV;
-      if ((o & QSF_OUT_FLUX) && pd.nborders > 0) {
-        double C[3];
-        coup.values(C);
-        // the flux time integral accumulates on the device, as on the fused path
-        g.flux(couples() == QSF_REP_P ? C : nullptr, pd.borders, pd.nborders, &row[7], fluxint.as<double>(), dt);
-      }
-      if (o & QSF_OUT_EKIN) {
-        g.fourier(QSF_REP_P);
-        double r[3];
-        g.observe(false, true, r);
-        row[4] = ekin = r[2] * g.dVm;
-        g.fourier(QSF_REP_X);
-      }
-      if (o & QSF_OUT_ETOT) row[5] = epot + ekin;
-      if (o & QSF_OUT_EDIFF) {
-        const double curr = epot + ekin;
-        row[6] = curr - last_change;
-        dif_energy = curr - last_change;
-        last_change = curr;
-      }
-      rows.insert(rows.end(), row.begin(), row.end());
-      return;
+    Grid& g = main();
+    if (o & QSF_OUT_NORMALIZE) g.normalize();
+    double r3[3] = {nan, nan, nan};
+    if (o & (QSF_OUT_NORM | QSF_OUT_EPOT)) g.observe((o & QSF_OUT_EPOT) != 0, false, r3);
+    if (o & QSF_OUT_NORM) row[2] = r3[0] * g.dV;
+    double epot = nan, ekin = nan;
+    if (o & QSF_OUT_EPOT) row[3] = epot = r3[1] * g.dV;
+    if ((o & QSF_OUT_FLUX) && pd.nborders > 0) {
+      double C[3];
+      coup.values(C);
+      // the flux time integral accumulates on the device, as on the fused path
+      g.flux(couples() == QSF_REP_P ? C : nullptr, pd.borders, pd.nborders, &row[7], fluxint.as<double>(), dt);
     }
-    // fused: the values come from the next pass over the main grid
+    if (o & QSF_OUT_EKIN) {
+      g.fourier(QSF_REP_P);
+      double r[3];
+      g.observe(false, true, r);
+      row[4] = ekin = r[2] * g.dVm;
+      g.fourier(QSF_REP_X);
+    }
+    if (o & QSF_OUT_ETOT) row[5] = epot + ekin;
+    if (o & QSF_OUT_EDIFF) {
+      const double curr = epot + ekin;
+      row[6] = curr - last_change;
+      dif_energy = curr - last_change;
+      last_change = curr;
+    }
+    rows.insert(rows.end(), row.begin(), row.end());
+  }
+
+  // the row of a fused step: its values come from the next pass over the main grid
+  void request_row(const Plan& plan) {
+    const std::vector<double> row = empty_row(plan.step, plan.timer);
     const int ri = (int)(rows.size() / width);
     rows.insert(rows.end(), row.begin(), row.end());
     if (devrec_used >= devrec_cap) {
@@ -1579,14 +1691,15 @@ struct Prop {
     }
     pend_obs = true;
     pend_row = (int)devrec_used++;
-    pend_ekin = (o & (QSF_OUT_EKIN | QSF_OUT_ETOT)) != 0;
-    coup.values(pend_obs_C);
+    pend_ekin = (pd.outputs & (QSF_OUT_EKIN | QSF_OUT_ETOT)) != 0;
+    std::copy(plan.C, plan.C + 3, pend_obs_C);
     pending_rows.push_back({ri, pend_ekin});
   }
 
   void sync_rows() {
     if (pending_rows.empty()) return;
     if (pend_obs) flush_obs_only();
+    drain_rows();
     std::vector<double> dev((size_t)devrec_used * kRecWidth);
     QSF_HIP(hipMemcpyAsync(dev.data(), devrec.p, dev.size() * sizeof(double), hipMemcpyDeviceToHost, st()));
     QSF_HIP(hipStreamSynchronize(st()));
@@ -1664,9 +1777,7 @@ struct Prop {
       coup.values(c3);
       after.C[s] = cx ? 0.0 : c3[0];
       if (o) {
-        std::vector<double> row(width, std::nan(""));
-        row[0] = (double)step;
-        row[1] = timer;
+        const std::vector<double> row = empty_row(step, timer);
         pending_rows.push_back({(int)(rows.size() / width), ekin});
         rows.insert(rows.end(), row.begin(), row.end());
       }
@@ -1809,17 +1920,8 @@ struct Prop {
 
   void compute_each() {
     if (pd.outputs == 0) return;
-    if (fused() && step > 0) request_row(true);
-    else {
-      if (fused()) flush();
-      request_row(false);
-    }
-  }
-
-  void make_step() {
-    auto ops = schedule();
-    if (fused()) exec_fused(ops);
-    else exec_simple(ops);
+    if (fused()) flush();
+    request_row();
   }
 
   void post_compute() {
@@ -1844,7 +1946,11 @@ struct Prop {
       line_steps(1);
       return;
     }
-    make_step();
+    if (fused()) {
+      run_fused(1);
+      return;
+    }
+    exec_simple(schedule());
     compute_each();
     post_compute();
   }
@@ -2606,6 +2712,10 @@ int qsf_prop_run_steps(qsf_prop* p, int64_t k, int64_t* done) {
     while (i < k && p->p.should_continue()) {
       if (p->p.line_path()) {
         i += p->p.line_steps(std::min(k - i, p->p.steps_left()));
+      } else if (p->p.fused()) {
+        const int64_t n = std::min(k - i, p->p.steps_left());
+        p->p.run_fused(n);
+        i += n;
       } else {
         p->p.loop_body();
         ++i;
