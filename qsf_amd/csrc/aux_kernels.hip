@@ -59,6 +59,28 @@ __global__ void pair_table_kernel(PairTableArgs a) {
   reinterpret_cast<T*>(a.out)[k] = T{(Real)re, (Real)im};
 }
 
+__global__ void potential_kernel(double* out, int64_t n, int64_t n1, int model, double xmin, double dx, double charge,
+                                 double soft) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n * n1) return;
+  if (model == QSF_POT_COULOMB) {
+    const double x = xmin + k * dx;
+    out[k] = charge / sqrt(x * x + soft);
+  } else if (model == QSF_POT_EBERLY) {
+    const double d = (double)k * dx;
+    out[k] = charge / sqrt(d * d + soft);
+  } else {
+    const double x = xmin + (k / n1) * dx, y = xmin + (k % n1) * dx;
+    out[k] = charge / sqrt((x - y) * (x - y) + x * y + soft);
+  }
+}
+
+void launch_potential(double* out, int64_t n, int64_t n1, int model, double xmin, double dx, double charge, double soft,
+                      hipStream_t s) {
+  hipLaunchKernelGGL(potential_kernel, dim3((unsigned)((n * n1 + 255) / 256)), dim3(256), 0, s, out, n, n1, model, xmin,
+                     dx, charge, soft);
+}
+
 template <typename Real>
 __global__ void radial_x_kernel(RadialArgs a) {
   using T = typename cvec<Real>::T;

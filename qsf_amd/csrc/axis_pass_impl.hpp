@@ -63,15 +63,20 @@ constexpr int var_wshift(int v) { return v % 3 == 0 ? 0 : (v % 3 == 1 ? -1 : 1);
 // contains, so passes that only transform and multiply by the P factor (the column passes, the
 // middle passes, plain transforms) run a build without the X stage, the observation, the flux
 // gather, the region mask and the multigrid edge writes: far fewer registers, more waves.
-// Row passes that carry the X halves and an observation but no region mask, multigrid edges or
-// kinetic-energy copy (the 3D step's last-axis pass) run a middle tier without those paths.
-enum PassFeat : int { FEAT_FULL = 0, FEAT_LEAN = 1, FEAT_X = 2 };
+// Passes that carry the X halves and an observation run a middle tier. Four more keep what the middle
+// tier would pay registers for (at 320 points FP64, with the boundary forms in it, its row pass fell
+// from two waves per SIMD to one, 252 -> 860 us at 320^3): the more tier takes several substeps of a
+// grid's one transformed axis, the boundary tier forms the state between the halves explicitly (it is copied, kept
+// or its transform is summed), the full tier also masks it and writes the multigrid edges (both
+// rows only), and the kinetic tier only transforms and sums.
+enum PassFeat : int { FEAT_FULL = 0, FEAT_LEAN = 1, FEAT_X = 2, FEAT_BOUNDARY = 3, FEAT_KIN = 4, FEAT_MORE = 5 };
 constexpr uint32_t kLeanFlags = F_INV1 | F_FWD | F_P | F_INV2 | F_SCALE | F_NOSTORE;
-constexpr uint32_t kXFlags = kLeanFlags | F_XA | F_XB | F_OBS;
-inline int feat_of(const PassParams& p, bool row) {
-  if ((p.flags & ~kLeanFlags) == 0 && !p.er_out) return FEAT_LEAN;
-  if (row && (p.flags & ~kXFlags) == 0 && !p.er_out && !((p.flags & F_OBS) && p.obs.copy_out)) return FEAT_X;
-  return FEAT_FULL;
+inline int feat_of(const PassParams& p) {
+  if ((p.flags & ~kLeanFlags) == 0 && !p.er_out && !p.nmore) return FEAT_LEAN;
+  if ((p.flags & F_OBS) && p.obs.kin_only) return FEAT_KIN;
+  if ((p.flags & F_MASK) || p.er_out) return FEAT_FULL;
+  if ((p.flags & (F_KEEP | F_KIN)) || ((p.flags & F_OBS) && (p.obs.copy_out || p.obs.want_epot))) return FEAT_BOUNDARY;
+  return p.nmore ? FEAT_MORE : FEAT_X;
 }
 
 // Block geometry per (precision, N, mode, variant).
@@ -200,39 +205,62 @@ template <int N> struct XEval {
   __device__ __forceinline__ T at(int n) const { return npr ? cmul(base_at(n), pair_at(n)) : base_at(n); }
 };
 
-__device__ __forceinline__ double pot_value(const ObsParams& o, const double* c, int D) {
-  // closed forms of potential.h (full or partial by free axes), evaluated in FP64
-  auto Ne = [&](double x) { return o.NE / sqrt(x * x + o.Nsoft); };
-  auto ee = [&](double x, double y) {
-    if (o.pot_kind == 3) return o.EE / sqrt((x - y) * (x - y) + x * y + o.Esoft);
-    return o.EE / sqrt((x - y) * (x - y) + o.Esoft);
-  };
-  const int fm = o.free_mask;
-  auto b = [&](int d) { return !(fm & (1 << d)); };
-  if (o.pot_kind == 0) return 0.0;
-  if (o.pot_kind == 1) {  // Coulomb over the bounded coordinates
-    double s = 0.0;
-    for (int d = D - 1; d >= 0; --d)
-      if (b(d)) s = c[d] * c[d] + s;
-    bool any = false;
-    for (int d = 0; d < D; ++d) any = any || b(d);
-    return any ? o.NE / sqrt(s + o.Nsoft) : 0.0;
+// Potential of the elements of one transform along `axis`, from its tables: the bounded axes'
+// electron-nucleus terms and the pair terms of potential.h:130-179 (evaluated once per table entry:
+// six square roots and divisions a point on a 3D grid otherwise). CoulombInteraction over several
+// bounded coordinates (:40-44) has no such tables and takes its closed form.
+struct PotEval {
+  double cst, rs;
+  const double* ax;
+  const double* pr0;
+  const double* pr1;
+  int o0, o1, npr, kind;
+  __device__ __forceinline__ void init(const ObsParams& o, int axis, int i0, int i1, int i2) {
+    auto id = [&](int d) { return d == 0 ? i0 : (d == 1 ? i1 : i2); };
+    cst = rs = 0.0;
+    ax = axis == 0 ? o.pot_axis[0] : (axis == 1 ? o.pot_axis[1] : o.pot_axis[2]);
+    npr = o0 = o1 = 0;
+    pr0 = pr1 = nullptr;
+    kind = o.pot_pair_kind;
+#pragma unroll
+    for (int d = 2; d >= 0; --d) {
+      if (d == axis) continue;
+      if (o.pot_axis[d]) cst += o.pot_axis[d][id(d)];
+      if (o.pot_radial && !(o.free_mask & (1 << d))) {
+        const double x = o.xmin[d] + id(d) * o.dx[d];
+        rs = x * x + rs;
+      }
+    }
+    if (kind != PAIR_NONE) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        if (!(o.pot_pair_mask & (1 << k))) continue;
+        const int p = k, q = (k + 1) % 3;   // pairs (0,1), (1,2), (2,0)
+        if (p != axis && q != axis) {
+          cst += o.pot_pair[kind == PAIR_DIFF ? (int64_t)abs(id(p) - id(q)) : (int64_t)id(p) * o.pot_pair_n + id(q)];
+        } else {
+          const int other = (p == axis) ? id(q) : id(p);
+          const double* base = o.pot_pair + (kind == PAIR_FULL ? (int64_t)other * o.pot_pair_n : 0);
+          if (npr == 0) { pr0 = base; o0 = other; }
+          else { pr1 = base; o1 = other; }
+          ++npr;
+        }
+      }
+    }
   }
-  double v = 0.0;
-  if (D == 1) return b(0) ? Ne(c[0]) : 0.0;
-  if (D == 2) {
-    if (b(0) && b(1)) v = ee(c[0], c[1]);
-    if (b(0)) v += Ne(c[0]);
-    if (b(1)) v += Ne(c[1]);
+  __device__ __forceinline__ double at(const ObsParams& o, int axis, int n) const {
+    double v = cst;
+    if (ax) v += ax[n];
+    if (npr > 0) v += kind == PAIR_DIFF ? pr0[abs(n - o0)] : pr0[n];
+    if (npr > 1) v += kind == PAIR_DIFF ? pr1[abs(n - o1)] : pr1[n];
+    if (o.pot_radial) {
+      const double x = (axis == 0 ? o.xmin[0] : (axis == 1 ? o.xmin[1] : o.xmin[2])) +
+                       n * (axis == 0 ? o.dx[0] : (axis == 1 ? o.dx[1] : o.dx[2]));
+      v += o.NE / sqrt((o.free_mask & (1 << axis) ? 0.0 : x * x) + rs + o.Nsoft);
+    }
     return v;
   }
-  if (b(0) && b(1)) v += ee(c[0], c[1]);
-  if (b(1) && b(2)) v += ee(c[1], c[2]);
-  if (b(2) && b(0)) v += ee(c[2], c[0]);
-  for (int d = 0; d < 3; ++d)
-    if (b(d)) v += Ne(c[d]);
-  return v;
-}
+};
 
 // Geometry of one thread's transform in tile b: (outer o, inner c), its global offsets and the
 // grid coordinates of its line (the transform axis index is per element).
@@ -319,7 +347,7 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
 
   // this thread's twiddles for every transform of the pass, and the flux gather's row range,
   // read with the state
-  Twiddles<N, ALT, T, FEAT == FEAT_LEAN, !ROW> tw;   // FP32 column tiles read twiddles directly
+  Twiddles<N, ALT, T, FEAT == FEAT_LEAN || FEAT == FEAT_KIN, !ROW> tw;   // FP32 column tiles read twiddles directly
   if (p.flags & (F_INV1 | F_FWD | F_INV2)) tw.load(roots, t);
   int gk0 = 0, gk1 = 0;
   if (FEAT != FEAT_LEAN && ROW && (p.flags & F_OBS) && p.obs.gather_rowptr && valid) {
@@ -330,12 +358,15 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
   if (p.flags & F_SCALE) {
     // the scale (1/m of an inverse transform: 1/768 has no exact FP32 form) is applied in FP64
     // with one rounding; a once-rounded FP32 scale would bias the norm the same way every step
+    const double sc = p.scale_dev ? p.scale * *p.scale_dev : p.scale;
 #pragma unroll
-    for (int q = 0; q < E; ++q) v[q] = capply(v[q], double2{p.scale, 0.0});
+    for (int q = 0; q < E; ++q) v[q] = capply(v[q], double2{sc, 0.0});
   }
 
+  int tx = t;
   auto run_fft = [&](auto dir_tag) {
     constexpr int DIR = decltype(dir_tag)::value;
+    const int t = tx;
     if constexpr (ROW) {
       RowAddr<T, Geo<Real, N, ROW, V>::WAVE_LINES> a{w * row_stride<T, N>()};
       fft<N, ALT, DIR>(v, t, lds, a, roots, tw);
@@ -349,11 +380,25 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
 
   if (p.flags & F_INV1) run_fft(INV{});
 
+  if constexpr (FEAT == FEAT_KIN) {
+    const double* kw = p.axis == 0 ? p.obs.kin_w[0] : (p.axis == 1 ? p.obs.kin_w[1] : p.obs.kin_w[2]);
+    double ek = 0.0;
+    if (valid) {
+#pragma unroll
+      for (int q = 0; q < E; ++q)
+        ek += ((double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y) * kw[t + TT * q];
+    }
+    for (int off = 32; off > 0; off >>= 1) ek += __shfl_xor(ek, off);
+    double* red = reinterpret_cast<double*>(smem_raw + G::red_off);
+    if ((tid & 63) == 0) { red[3 * (tid >> 6)] = 0.0; red[3 * (tid >> 6) + 1] = 0.0; red[3 * (tid >> 6) + 2] = ek; }
+    return;
+  }
+
   // X stage: A factor -> observables / region mask -> B factor, one loop over the elements.
   // When both halves use the same pair-interaction table its lookup is shared.
-  const uint32_t XF = FEAT != FEAT_LEAN ? p.flags & (F_XA | F_OBS | F_MASK | F_XB) : 0u;
+  const uint32_t XF = FEAT != FEAT_LEAN ? p.flags & (F_XA | F_OBS | (FEAT == FEAT_FULL ? F_MASK : 0u) | F_XB) : 0u;
   if (XF) {
-    const bool doA = p.flags & F_XA, doB = p.flags & F_XB, obs = p.flags & F_OBS, msk = p.flags & F_MASK;
+    const bool doA = p.flags & F_XA, doB = p.flags & F_XB, obs = p.flags & F_OBS, msk = FEAT == FEAT_FULL && (p.flags & F_MASK);
     XEval<N> xa, xb;
     if (doA) xa.init(p.xa, p.axis, i0, i1, i2);
     if (doB) xb.init(p.xb, p.axis, i0, i1, i2);
@@ -367,9 +412,11 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
     const ObsParams& ob = p.obs;
     double nrm = 0.0, ep = 0.0, ek = 0.0, kc = 0.0;
     const double* ka = nullptr;
-    int D = 1;
+    PotEval pot;
     if (obs) {
-      D = p.n[2] > 1 ? 3 : (p.n[1] > 1 ? 2 : 1);
+      if constexpr (FEAT == FEAT_BOUNDARY || FEAT == FEAT_FULL) {
+        if (ob.want_epot) pot.init(ob, p.axis, i0, i1, i2);
+      }
 #pragma unroll
       for (int d = 0; d < 3; ++d)
         if (d != p.axis && ob.kin_w[d]) kc += ob.kin_w[d][id(d)];
@@ -396,7 +443,9 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
     // it (the region mask, the multigrid edges, the copy for the kinetic energy). Otherwise both
     // halves meet in one product per element, the observables weight |psi|^2 by |A factor|^2,
     // and the flux gather keeps the state before A and applies A at the points it reads.
-    const bool compact = FEAT == FEAT_X || (!msk && !(ROW && p.er_out) && !(obs && ob.copy_out));
+    const bool keep = p.flags & F_KEEP;
+    const bool compact = FEAT == FEAT_X || FEAT == FEAT_MORE ||
+                         (FEAT == FEAT_BOUNDARY && !keep && !(obs && ob.copy_out));
     if (compact) {
 #pragma unroll
       for (int q = 0; q < E; ++q) {
@@ -421,19 +470,15 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
         if (obs && valid) {
           const double a2 = ((double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y) * wa;
           nrm += a2;
-          if (ob.want_epot) {
-            double co[3];
-            co[0] = ob.xmin[0] + (p.axis == 0 ? ia : i0) * ob.dx[0];
-            co[1] = ob.xmin[1] + (p.axis == 1 ? ia : i1) * ob.dx[1];
-            co[2] = ob.xmin[2] + (p.axis == 2 ? ia : i2) * ob.dx[2];
-            ep += a2 * pot_value(ob, co, D);
+          if constexpr (FEAT == FEAT_BOUNDARY) {
+            if (ob.want_epot) ep += a2 * pot.at(ob, p.axis, ia);
           }
           if (ka || kc != 0.0) ek += a2 * (kc + (ka ? ka[ia] : 0.0));
         }
         if (gline) glds[w * G::gather_stride + ia] = v[q];
         if (doA || doB) v[q] = capply(v[q], zab);
       }
-    } else if constexpr (FEAT == FEAT_FULL) {
+    } else if constexpr (FEAT == FEAT_BOUNDARY || FEAT == FEAT_FULL) {
 #pragma unroll
     for (int q = 0; q < E; ++q) {
       const int ia = t + TT * q;
@@ -446,17 +491,13 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
       if (obs && valid) {
         const double a2 = (double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y;
         nrm += a2;
-        if (ob.want_epot) {
-          double co[3];
-          co[0] = ob.xmin[0] + (p.axis == 0 ? ia : i0) * ob.dx[0];
-          co[1] = ob.xmin[1] + (p.axis == 1 ? ia : i1) * ob.dx[1];
-          co[2] = ob.xmin[2] + (p.axis == 2 ? ia : i2) * ob.dx[2];
-          ep += a2 * pot_value(ob, co, D);
-        }
+        if (ob.want_epot) ep += a2 * pot.at(ob, p.axis, ia);
         if (ka || kc != 0.0) ek += a2 * (kc + (ka ? ka[ia] : 0.0));
         if (ob.copy_out) reinterpret_cast<S*>(ob.copy_out)[base + (int64_t)ia * step] = to_state<S>(v[q]);
       }
+      if (keep && valid) dst[base + (int64_t)ia * step] = to_state<S>(v[q]);
       if (gline) glds[w * G::gather_stride + ia] = v[q];
+      if constexpr (FEAT == FEAT_FULL) {
       if (ROW && p.er_out && valid) {
         // multigrid source edges of the boundary state (2D main region, row i0 = o)
         const int64_t nc = p.nCAP, n0 = p.n[0], n1 = N;
@@ -480,6 +521,7 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
         }
         const double mk = p.mask_tab[off];
         v[q] = T{(Real)((double)v[q].x * mk), (Real)((double)v[q].y * mk)};
+      }
       }
       if (doB) v[q] = capply(v[q], same ? za : (shared ? cmul(xb.base_at(ia), pp) : xb.at(ia)));
     }
@@ -512,25 +554,62 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
     }
   }
 
-  if (p.flags & F_FWD) run_fft(FWD{});
-
-  if (p.flags & F_P) {
-    // P phase: complex FP64 per-axis tables, one FP64 product per element
-    double2 cst{1.0, 0.0};
-    if (p.axis != 0 && pf0) cst = cmul(cst, ld<double2>(pf0, i0));
-    if (p.axis != 1 && pf1) cst = cmul(cst, ld<double2>(pf1, i1));
-    if (p.axis != 2 && pf2) cst = cmul(cst, ld<double2>(pf2, i2));
-    const double2* pa = reinterpret_cast<const double2*>(p.axis == 0 ? pf0 : (p.axis == 1 ? pf1 : pf2));
+  // forward transform, P factor, inverse transform; a pass along the only transformed axis of its
+  // grid takes its further substeps here too, the state staying in registers between them
+  for (int sub = 0;; ++sub) {   // (one round in every tier but the more tier)
+    if constexpr (FEAT == FEAT_MORE) {
+      // (opaque: the loop would otherwise keep every exchange address of both transforms in registers)
+      asm volatile("" : "+v"(tx));
+      if (sub > 0) {
+        if constexpr (!std::is_same_v<S, T>) {
 #pragma unroll
-    for (int q = 0; q < E; ++q) {
-      const double2 f = pa ? cmul(cst, pa[t + TT * q]) : cst;
-      v[q] = capply(v[q], f);
+          for (int q = 0; q < E; ++q) v[q] = from_state<T>(to_state<S>(v[q]));   // rounded as a pass stores it
+        }
+        XEval<N> x;
+        x.init(p.more[sub - 1].x, p.axis, i0, i1, i2);
+#pragma unroll
+        for (int q = 0; q < E; ++q) v[q] = capply(v[q], x.at(t + TT * q));
+      }
     }
+    if (p.flags & F_FWD) run_fft(FWD{});
+
+    if constexpr (FEAT == FEAT_BOUNDARY) {
+      if (p.flags & F_KIN) {
+        double ek = 0.0;
+        if (valid) {
+#pragma unroll
+          for (int q = 0; q < E; ++q)
+            ek += ((double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y) * p.obs.kin_fwd[t + TT * q];
+        }
+        for (int off = 32; off > 0; off >>= 1) ek += __shfl_xor(ek, off);
+        // beside the wave's other sums, which the observation left there
+        if ((tid & 63) == 0) reinterpret_cast<double*>(smem_raw + G::red_off)[3 * (tid >> 6) + 2] = ek;
+      }
+    }
+
+    if (p.flags & F_P) {
+      // P phase: complex FP64 per-axis tables, one FP64 product per element
+      const bool first = FEAT != FEAT_MORE || sub == 0;
+      const void* f0 = first ? pf0 : p.more[sub - 1].pf[0];
+      const void* f1 = first ? pf1 : p.more[sub - 1].pf[1];
+      const void* f2 = first ? pf2 : p.more[sub - 1].pf[2];
+      double2 cst{1.0, 0.0};
+      if (p.axis != 0 && f0) cst = cmul(cst, ld<double2>(f0, i0));
+      if (p.axis != 1 && f1) cst = cmul(cst, ld<double2>(f1, i1));
+      if (p.axis != 2 && f2) cst = cmul(cst, ld<double2>(f2, i2));
+      const double2* pa = reinterpret_cast<const double2*>(p.axis == 0 ? f0 : (p.axis == 1 ? f1 : f2));
+#pragma unroll
+      for (int q = 0; q < E; ++q) {
+        const double2 f = pa ? cmul(cst, pa[t + TT * q]) : cst;
+        v[q] = capply(v[q], f);
+      }
+    }
+
+    if (p.flags & F_INV2) run_fft(INV{});
+    if (FEAT != FEAT_MORE || sub >= p.nmore) break;
   }
 
-  if (p.flags & F_INV2) run_fft(INV{});
-
-  if (valid && !(p.flags & F_NOSTORE)) {
+  if (valid && !(p.flags & (F_NOSTORE | F_KEEP))) {
 #pragma unroll
     for (int q = 0; q < E; ++q) dst[base + (int64_t)(t + TT * q) * step] = to_state<S>(v[q]);
   }
@@ -548,8 +627,9 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
 // uncapped.
 template <int E, int FEAT, bool UNIFORM_LINE>
 constexpr int pass_waves() {
-  if (E <= 8) return (FEAT == FEAT_LEAN || UNIFORM_LINE) ? 4 : 3;
-  if (E <= 16) return FEAT == FEAT_LEAN ? 3 : 2;   // (the X tier counts as full)
+  constexpr bool light = FEAT == FEAT_LEAN || FEAT == FEAT_KIN;
+  if (E <= 8) return (light || UNIFORM_LINE) ? 4 : 3;
+  if (E <= 16) return light ? 3 : 2;   // (the X tier counts as full)
   return 1;
 }
 
@@ -563,6 +643,7 @@ __global__ void __launch_bounds__((Geo<Real, N, ROW, V>::THREADS),
   constexpr int E = PL::E, TT = PL::T;
   constexpr int W = Geo<Real, N, ROW, V>::W;
   extern __shared__ __align__(16) unsigned char smem_raw[];
+  if (p.halt && *p.halt) return;   // (the whole grid: the flag changes only between passes)
 
   const int tid = threadIdx.x;
   const int t = ROW ? (tid % TT) : (tid / W);
@@ -652,12 +733,20 @@ inline int launch_feat(const PassParams& p, hipStream_t s) {
 
 template <typename Real, int N, bool ROW, int V, bool S32>
 inline int launch_one(const PassParams& p, hipStream_t s) {
-  const int f = feat_of(p, ROW);
+  const int f = feat_of(p);
   if (f == FEAT_LEAN) return launch_feat<Real, N, ROW, V, FEAT_LEAN, S32>(p, s);
-  if constexpr (ROW) {
-    if (f == FEAT_X) return launch_feat<Real, N, ROW, V, FEAT_X, S32>(p, s);
+  if (f == FEAT_X) return launch_feat<Real, N, ROW, V, FEAT_X, S32>(p, s);
+  if (f == FEAT_KIN) return launch_feat<Real, N, ROW, V, FEAT_KIN, S32>(p, s);
+  if (f == FEAT_MORE) {
+    if constexpr (S32) return -1;   // (an FP32 state under FP64 arithmetic has no regions)
+    else return launch_feat<Real, N, ROW, V, FEAT_MORE, S32>(p, s);
   }
-  return launch_feat<Real, N, ROW, V, FEAT_FULL, S32>(p, s);
+  if constexpr (ROW) {
+    if (f == FEAT_BOUNDARY) return launch_feat<Real, N, ROW, V, FEAT_BOUNDARY, S32>(p, s);
+    return launch_feat<Real, N, ROW, V, FEAT_FULL, S32>(p, s);
+  } else {
+    return -1;   // masks, edges and formed boundaries are the row passes' work
+  }
 }
 
 // Blocks of a launch, which is also the number of per-block observation sums it writes.

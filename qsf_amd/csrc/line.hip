@@ -46,18 +46,6 @@ void launch_line_tables(const AxisTableArgs& a, const LineCouplings& c, int tabl
                      0, s, a, c);
 }
 
-// The potential of a line's nodes (what pot_value gives the observation passes in 1D).
-__global__ void line_potential_kernel(double* out, int64_t n, ObsParams o) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double co[3] = {o.xmin[0] + i * o.dx[0], 0.0, 0.0};
-  out[i] = pot_value(o, co, 1);
-}
-
-void launch_line_potential(double* out, int64_t n, const ObsParams& o, hipStream_t s) {
-  hipLaunchKernelGGL(line_potential_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, out, n, o);
-}
-
 // One wave per step: the step's sums over the line kernel's waves and its fluxes, in fixed order.
 template <typename Real>
 __global__ void line_rows_kernel(LineRows a, LineCouplings c) {

@@ -17,7 +17,9 @@ enum PassFlags : uint32_t {
   F_INV2 = 1u << 6,     // inverse transform after the P factor
   F_SCALE = 1u << 7,    // multiply by `scale` at load
   F_MASK = 1u << 8,     // multiply by the region mask (after observing, before the B factor)
-  F_NOSTORE = 1u << 9   // read-only pass (observables only)
+  F_NOSTORE = 1u << 9,  // read-only pass (observables only)
+  F_KEEP = 1u << 10,    // store the observed state (after the A factor), not the pass's end
+  F_KIN = 1u << 11      // kinetic sum of the forward transform (obs.kin_fwd), into the third sum
 };
 
 // Pair interaction part of an X factor: none, a table indexed by |i-j| (Eberly), or a full n*n
@@ -41,11 +43,18 @@ struct XFactor {
 struct ObsParams {
   double* partials;      // per block: [norm, epot, ekin]
   const double* kin_w[3];  // per-axis additive weights for <½p²> (nullptr = 0)
-  // potential for <V> (closed forms of potential.h evaluated on the fly)
-  int32_t pot_kind, free_mask;
-  double NE, EE, Nsoft, Esoft;
+  const double* kin_fwd; // F_KIN: weights over the transform axis
+  // potential for <V>: per-axis tables (electron-nucleus) and a pair table laid out as an X factor's,
+  // or, for CoulombInteraction over two or more bounded coordinates, its closed form per point
+  const double* pot_axis[3];
+  const double* pot_pair;
+  int32_t pot_pair_kind, pot_pair_mask;
+  int64_t pot_pair_n;
+  int32_t pot_radial, free_mask;
+  double NE, Nsoft;
   double xmin[3], dx[3];
   int32_t want_epot;
+  int32_t kin_only;        // a read-only pass that only sums kin_w over the transform axis
   // sparse gather of the points flux needs (row-major rows of the last axis)
   const int32_t* gather_rowptr;   // rows+1
   const int32_t* gather_pos;      // position within the row of each gathered point
@@ -63,6 +72,13 @@ struct BatchEntry {
   int64_t total_steps;     // steps the solve takes; later steps of the batch skip it
 };
 
+// A further substep of a pass along the one transformed axis of a grid.
+struct MoreSub {
+  XFactor x;
+  const void* pf[3];
+};
+constexpr int kMoreSubs = 3;
+
 struct PassParams {
   const BatchEntry* batch; // non-null: batched launch, per-solve pointers from batch[blockIdx.y]
   const int64_t* step_ctr; // device step counter of a batched launch
@@ -77,8 +93,12 @@ struct PassParams {
   const void* roots;     // N roots exp(-2πi j/N)
   uint32_t flags;
   double scale;
+  const double* scale_dev; // F_SCALE: a device factor on top of `scale`, or nullptr
+  const int32_t* halt;     // the pass does nothing once this is non-zero (nullptr: always runs)
   XFactor xa, xb;
   const void* pf[3];     // P factor tables (n_a entries; nullptr = 1)
+  int32_t nmore;         // further substeps [X, forward, P, inverse] after the first, at most kMoreSubs
+  MoreSub more[kMoreSubs];
   ObsParams obs;
   // region mask (F_MASK): FP64 table over per-axis CAP nodes clamped to [0, nCAP]
   const double* mask_tab;

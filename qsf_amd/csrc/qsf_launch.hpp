@@ -69,6 +69,11 @@ struct PairTableArgs {
 };
 void launch_pair_table(int precision, const PairTableArgs& a, hipStream_t s);
 
+// Potential tables (FP64): model QSF_POT_COULOMB: charge / sqrt(x_i^2 + soft), n entries; Eberly: by
+// |i-j|, n entries; Eckhardt-Sacha: n * n1 entries (potential.h:130-179).
+void launch_potential(double* out, int64_t n, int64_t n1, int model, double xmin, double dx, double charge, double soft,
+                      hipStream_t s);
+
 // psi *= exp(-i delta V) (RE) or exp(-delta V) (IM) with V = NE / sqrt(sum x_d^2 + Nsoft) over the
 // bounded coordinates (CoulombInteraction, potential.h:40-44), in place on an X-rep state.
 struct RadialArgs {
@@ -151,7 +156,6 @@ struct LineCouplings {
 // `tables` tables of a.n entries at a.out, table k with coupling c.C[k] and substep length
 // c.delta[k % c.per_step].
 void launch_line_tables(const AxisTableArgs& a, const LineCouplings& c, int tables, hipStream_t s);
-void launch_line_potential(double* out, int64_t n, const ObsParams& o, hipStream_t s);
 struct LineRows {
   const double* sums;
   int32_t waves, nvals;

@@ -11,14 +11,15 @@
 
 namespace qsf {
 
-// Norm and potential sums of slot blockIdx.y: block x takes chunk x of the slot's tiles (one chunk
-// of all tiles where they are few).
+// The first NC sums of slot blockIdx.y: block x takes chunk x of the slot's tiles (one chunk of all
+// tiles where they are few).
+template <int NC>
 __global__ void rows_reduce_kernel(const double* in, int64_t slot_stride, int64_t count, int width, int64_t chunk,
                                    double* out, int64_t out_stride) {
   __shared__ double red[256];
   const double* p = in + (int64_t)blockIdx.y * slot_stride;
   const int64_t lo = (int64_t)blockIdx.x * chunk, hi = lo + chunk < count ? lo + chunk : count;
-  for (int c = 0; c < 2; ++c) {
+  for (int c = 0; c < NC; ++c) {
     double acc = 0.0;
     for (int64_t k = lo + threadIdx.x; k < hi; k += 256) acc += p[k * width + c];
     red[threadIdx.x] = acc;
@@ -27,7 +28,7 @@ __global__ void rows_reduce_kernel(const double* in, int64_t slot_stride, int64_
       if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
       block_sync();
     }
-    if (threadIdx.x == 0) out[(int64_t)blockIdx.y * out_stride + blockIdx.x * 2 + c] = red[0];
+    if (threadIdx.x == 0) out[(int64_t)blockIdx.y * out_stride + blockIdx.x * NC + c] = red[0];
     block_sync();
   }
 }
@@ -106,17 +107,23 @@ int flux_blocks(int64_t npts) {
   return (int)(want < 1 ? 1 : (want > 1024 ? 1024 : want));
 }
 
-void launch_rows(int precision, const RowSlots& a, int slots, hipStream_t s) {
-  if (a.tiles <= 4096) {
-    hipLaunchKernelGGL(rows_reduce_kernel, dim3(1, (unsigned)slots), dim3(256), 0, s, a.partials, a.tiles * 3, a.tiles, 3,
-                       a.tiles, a.rec, a.rec_width);
-  } else {
-    const int64_t chunk = (a.tiles + 255) / 256;
-    hipLaunchKernelGGL(rows_reduce_kernel, dim3(256, (unsigned)slots), dim3(256), 0, s, a.partials, a.tiles * 3, a.tiles,
-                       3, chunk, a.scratch, (int64_t)512);
-    hipLaunchKernelGGL(rows_reduce_kernel, dim3(1, (unsigned)slots), dim3(256), 0, s, (const double*)a.scratch,
-                       (int64_t)512, (int64_t)256, 2, (int64_t)256, a.rec, a.rec_width);
+template <int NC>
+static void reduce_slots(const RowSlots& a, const double* in, int64_t tiles, double* out, int slots, hipStream_t s) {
+  if (tiles <= 4096) {
+    hipLaunchKernelGGL(rows_reduce_kernel<NC>, dim3(1, (unsigned)slots), dim3(256), 0, s, in, tiles * 3, tiles, 3, tiles,
+                       out, a.rec_width);
+    return;
   }
+  const int64_t chunk = (tiles + 255) / 256;
+  hipLaunchKernelGGL(rows_reduce_kernel<NC>, dim3(256, (unsigned)slots), dim3(256), 0, s, in, tiles * 3, tiles, 3, chunk,
+                     a.scratch, (int64_t)512);
+  hipLaunchKernelGGL(rows_reduce_kernel<NC>, dim3(1, (unsigned)slots), dim3(256), 0, s, (const double*)a.scratch,
+                     (int64_t)512, (int64_t)256, NC, (int64_t)256, out, a.rec_width);
+}
+
+void launch_rows(int precision, const RowSlots& a, int slots, hipStream_t s) {
+  reduce_slots<2>(a, a.partials, a.tiles, a.rec, slots, s);
+  if (a.ktiles) reduce_slots<1>(a, a.kin + 2, a.ktiles, a.rec + 2, slots, s);
   if (a.flux.nb <= 0) return;
   const int blocks = flux_blocks(a.flux.npts);
   const dim3 grid((unsigned)blocks, (unsigned)slots);

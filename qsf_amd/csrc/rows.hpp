@@ -10,7 +10,9 @@ constexpr int kRowSlots = 32;   // boundaries one reduction takes
 struct RowSlots {
   const double* partials;    // [slot][tiles][3] block sums of the observing passes
   int64_t tiles;
-  double* rec;               // [slot][rec_width]: norm and potential sums, kinetic (not written), fluxes
+  const double* kin;         // [slot][ktiles][3] block sums of the kinetic passes (third sum)
+  int64_t ktiles;            // 0: no kinetic energy
+  double* rec;               // [slot][rec_width]: norm, potential and kinetic sums, fluxes
   int64_t rec_width;
   double* scratch;           // [slot][256 * 2] second reduction level (more than 4096 tiles)
   FluxArgs flux;             // nb = 0: no fluxes; gathered: [slot][nvals]; partials: [slot][blocks * nb]

@@ -190,7 +190,7 @@ struct Grid {
   std::vector<int> fftAxes;
   int pperm[3];
   DBuf psi, aux, partials, red, redscratch, kinw, masktab, invtab, corrtab, m1tab, tabs;
-  DBuf linetabs, linesums, linevals, linepot;   // workspaces of line runs (Prop::line_steps)
+  DBuf linetabs, linesums, linevals;   // workspaces of line runs (Prop::line_steps)
   int linehalf = 0;
   std::map<int64_t, std::unique_ptr<DBuf>> roots;
   std::map<std::pair<int64_t, int>, std::unique_ptr<DBuf>> pairs;
@@ -259,6 +259,7 @@ struct Grid {
     red.ensure(64 * sizeof(double));
     redscratch.ensure(256 * 16 * sizeof(double));
     build_static_tables();
+    build_potential();
   }
 
   hipStream_t st() const { return ctx->stream; }
@@ -297,15 +298,20 @@ struct Grid {
     // <½p²> weights per axis with the reference's P coordinates (coords.h:132-138; storage axis
     // parameters under the transposed layout)
     int64_t maxn = *std::max_element(n, n + 3);
-    kinw.ensure(3 * maxn * sizeof(double));
-    std::vector<double> kw(3 * maxn, 0.0);
+    // Behind them the weights of the kinetic sum taken axis by axis: sum_k w(k) |F psi|^2 over all axes
+    // is the sum over the axes a of (m / n_a) sum w_a(k_a) |F_a psi|^2 with the transform along a alone
+    // (Parseval along the others); for the forward transform, then for the inverse one (index -k).
+    std::vector<double> kw(9 * maxn, 0.0);
     for (int a = 0; a < D; ++a) {
       const int s = pperm[a];
       for (int64_t i = 0; i < n[a]; ++i) {
         const double p = dp[s] * (double)(i < n2[s] ? i : i - n[s]);
         kw[a * maxn + i] = 0.5 * p * p;
+        kw[(3 + a) * maxn + i] = 0.5 * p * p * (double)(m / n[a]);
+        kw[(6 + a) * maxn + (n[a] - i) % n[a]] = kw[(3 + a) * maxn + i];
       }
     }
+    kinw.ensure(kw.size() * sizeof(double));
     QSF_HIP(hipMemcpy(kinw.p, kw.data(), kw.size() * sizeof(double), hipMemcpyHostToDevice));
     if (d.absorber != QSF_ABS_NONE && d.nCAP > 0) {
       // region mask over clamped nodes of the bounded axes (grid.h:582-597)
@@ -505,16 +511,48 @@ struct Grid {
     return p;
   }
 
+  // Tables of the potential (FP64, n entries an axis and one pair table); the observation passes
+  // read them, also the one that may not allocate, so they are made with the grid.
+  DBuf pottabs;
+  int first_bounded() const {
+    int a = 0;
+    while (a < D && !bounded[a]) ++a;
+    return a;
+  }
+  bool potential_tables() const { return d.potential != QSF_POT_NONE && !radial; }
+  void build_potential() {
+    if (!potential_tables()) return;
+    const int64_t maxn = *std::max_element(n, n + 3);
+    const int f = first_bounded();
+    const int64_t n1 = d.potential == QSF_POT_EBERLY ? 1 : n[f];
+    pottabs.ensure((3 * maxn + (pair_mask() ? n[f] * n1 : 0)) * sizeof(double));
+    for (int a = 0; a < D; ++a)
+      if (bounded[a])
+        launch_potential(pottabs.as<double>() + a * maxn, n[a], 1, QSF_POT_COULOMB, xmin[a], dx[a],
+                         d.Ncharge * d.Echarge, d.Nsoft, st());
+    if (pair_mask())
+      launch_potential(pottabs.as<double>() + 3 * maxn, n[f], n1, d.potential, xmin[f], dx[f], d.Echarge * d.Echarge,
+                       d.Esoft, st());
+  }
+
   void obs_params(ObsParams& o, bool epot) {
-    o.pot_kind = d.potential == QSF_POT_COULOMB ? 1 : d.potential == QSF_POT_EBERLY ? 2
-               : d.potential == QSF_POT_ECKHARDT_SACHA ? 3 : 0;
     o.free_mask = freeMask;
     o.NE = d.Ncharge * d.Echarge;
-    o.EE = d.Echarge * d.Echarge;
     o.Nsoft = d.Nsoft;
-    o.Esoft = d.Esoft;
     for (int i = 0; i < 3; ++i) { o.xmin[i] = xmin[i]; o.dx[i] = dx[i]; }
     o.want_epot = epot;
+    if (!epot) return;
+    o.pot_radial = radial;
+    if (!potential_tables()) return;
+    const int64_t maxn = *std::max_element(n, n + 3);
+    for (int a = 0; a < D; ++a)
+      if (bounded[a]) o.pot_axis[a] = pottabs.as<double>() + a * maxn;
+    if (pair_mask()) {
+      o.pot_pair = pottabs.as<double>() + 3 * maxn;
+      o.pot_pair_kind = d.potential == QSF_POT_EBERLY ? PAIR_DIFF : PAIR_FULL;
+      o.pot_pair_mask = pair_mask();
+      o.pot_pair_n = n[first_bounded()];
+    }
   }
 
   void build_tables() {
@@ -683,6 +721,19 @@ struct Grid {
     launch_reduce_partials(partials.as<double>(), tiles, 3, red.as<double>(), redscratch.as<double>(), st());
     QSF_HIP(hipMemcpyAsync(host3, red.p, 3 * sizeof(double), hipMemcpyDeviceToHost, st()));
     QSF_HIP(hipStreamSynchronize(st()));
+  }
+
+  const double* kin_axis(int a, bool inverse) const {
+    return kinw.as<double>() + (size_t)((inverse ? 6 : 3) + a) * *std::max_element(n, n + 3);
+  }
+  // The read-only pass whose third block sums are axis a's part of the kinetic sum of X state `state`.
+  PassParams kinetic_pass(int a, void* state) {
+    PassParams q = params(a, state, state);
+    q.flags = F_INV1 | F_OBS | F_NOSTORE;
+    obs_params(q.obs, false);
+    q.obs.kin_w[a] = kin_axis(a, true);
+    q.obs.kin_only = 1;
+    return q;
   }
 
   double average(int R, int op) {
@@ -1409,24 +1460,32 @@ struct Prop {
 
   // ---- boundary observations: sums and flux stencils wait in slots and are reduced together ----
   bool fluxes() const { return pd.nborders > 0 && (pd.outputs & QSF_OUT_FLUX); }
-  int64_t slot_tiles = 0, slot_vals = 0;
+  int64_t slot_tiles = 0, slot_vals = 0, slot_ktiles = 0;
   int slot_cap = 0, slots = 0, slot_row = 0;   // slot k holds the boundary of record row slot_row + k
   double slot_C[kRowSlots][3];
-  DBuf slot_partials, slot_values, slot_scratch, slot_flux;
+  DBuf slot_partials, slot_values, slot_scratch, slot_flux, slot_kin;
 
   void ensure_slots(Grid& g, int64_t tiles) {
     const int64_t vals = fluxes() ? g.gather->nvals : 0;
-    if (slot_cap && tiles == slot_tiles && vals == slot_vals) return;
+    int64_t ktiles = 0;
+    if (pend_ekin)
+      for (int a : g.fftAxes) {
+        const PassParams q = g.kinetic_pass(a, g.psi.p);
+        ktiles += axis_pass_tiles(g.prec, q, g.variant(q));
+      }
+    if (slot_cap && tiles == slot_tiles && vals == slot_vals && ktiles == slot_ktiles) return;
     drain_rows();
     slot_tiles = tiles;
     slot_vals = vals;
+    slot_ktiles = ktiles;
     // 64 MiB of slots: all of them for planes, one or two for the largest cubes, whose single
     // boundary is work enough for the device
-    const int64_t bytes = tiles * 3 * (int64_t)sizeof(double) + vals * (int64_t)g.cb;
+    const int64_t bytes = (tiles + ktiles) * 3 * (int64_t)sizeof(double) + vals * (int64_t)g.cb;
     slot_cap = (int)std::max<int64_t>(1, std::min<int64_t>(kRowSlots, (int64_t(64) << 20) / std::max<int64_t>(bytes, 1)));
     slot_partials.ensure((size_t)slot_cap * tiles * 3 * sizeof(double));
     slot_values.ensure((size_t)slot_cap * std::max<int64_t>(vals, 1) * g.cb);
     slot_scratch.ensure((size_t)slot_cap * 512 * sizeof(double));
+    slot_kin.ensure((size_t)slot_cap * std::max<int64_t>(ktiles, 1) * 3 * sizeof(double));
     if (fluxes()) slot_flux.ensure((size_t)slot_cap * flux_blocks(g.gather->npts) * pd.nborders * sizeof(double));
   }
 
@@ -1436,6 +1495,8 @@ struct Prop {
     double* rec = devrec.as<double>() + (size_t)slot_row * kRecWidth;
     if (slots == 1) {   // one boundary: the single-row kernels, which finish its fluxes in fewer launches
       launch_reduce_partials(slot_partials.as<double>(), slot_tiles, 3, rec, slot_scratch.as<double>(), st(), 2);
+      if (slot_ktiles)
+        launch_reduce_partials(slot_kin.as<double>() + 2, slot_ktiles, 3, rec + 2, slot_scratch.as<double>(), st(), 1);
       if (fluxes()) {
         FluxArgs f = g.flux_args(slot_C[0], fluxint.as<double>(), dt);
         f.gathered = slot_values.p;
@@ -1449,6 +1510,8 @@ struct Prop {
       r.rec = rec;
       r.rec_width = kRecWidth;
       r.scratch = slot_scratch.as<double>();
+      r.kin = slot_kin.as<double>();
+      r.ktiles = slot_ktiles;
       r.nvals = slot_vals;
       if (fluxes()) {
         r.flux = g.flux_args(nullptr, fluxint.as<double>(), dt);
@@ -1479,30 +1542,20 @@ struct Prop {
     }
   }
 
-  double* obs_row() { return devrec.as<double>() + (size_t)pend_row * kRecWidth; }
-
   void after_obs(Grid& g) {
     // the boundary's sums and stencil stay in their slot until drain_rows
     if (!slots) slot_row = pend_row;
     for (int a = 0; a < 3; ++a) slot_C[slots][a] = couples() == QSF_REP_P ? pend_obs_C[a] : 0.0;
     ++slots;
-    double* rec = obs_row();
     if (pend_ekin) {
-      // kinetic energy: forward transform of the copied boundary state, then <½p²>
-      Grid& gg = g;
-      for (int a : gg.fftAxes) {
-        PassParams q = gg.params(a, gg.aux.p, gg.aux.p);
-        q.flags = F_FWD;
-        gg.run(q);
+      // kinetic energy of the copied boundary state: one read-only pass per axis
+      double* out = slot_kin.as<double>() + (size_t)(slots - 1) * slot_ktiles * 3;
+      for (int a : g.fftAxes) {
+        PassParams q = g.kinetic_pass(a, g.aux.p);
+        q.obs.partials = out;
+        out += 3 * axis_pass_tiles(g.prec, q, g.variant(q));
+        g.run(q);
       }
-      PassParams q = gg.params(gg.D - 1, gg.aux.p, gg.aux.p);
-      q.flags = F_OBS | F_NOSTORE;
-      gg.obs_params(q.obs, false);
-      int64_t maxn = *std::max_element(gg.n, gg.n + 3);
-      for (int a = 0; a < gg.D; ++a) q.obs.kin_w[a] = gg.kinw.as<double>() + a * maxn;
-      int t2 = gg.run(q);
-      // the kinetic column alone, straight into the record row (its norm and epot stay)
-      launch_reduce_partials(gg.partials.as<double>() + 2, t2, 3, rec + 2, gg.redscratch.as<double>(), st(), 1);
     }
   }
 
@@ -1794,12 +1847,6 @@ struct Prop {
       launch_line_tables(args(!cx, linestatic.p), fixed, still, st());
     }
     launch_line_tables(args(cx, mt), moving, (int)run * per, st());
-    if (!g.linepot.p) {
-      ObsParams ob{};
-      g.obs_params(ob, true);
-      g.linepot.ensure(N * sizeof(double));
-      launch_line_potential(g.linepot.as<double>(), N, ob, st());
-    }
     LineParams p{};
     const int var = ctx->variant_of(g.prec, 1, N, g.m);
     const int waves = launch_line(g.prec, N, var, p, st());
@@ -1815,7 +1862,9 @@ struct Prop {
     p.ptab = cx ? ft : mt;
     p.ptab_step = cx ? 0 : (int64_t)per * N;
     if (deferred[0] && pend[0].on) p.za_in = static_cast<const double2*>(pend[0].f.axis[0]);
-    p.vtab = g.linepot.as<double>();
+    ObsParams ob{};
+    g.obs_params(ob, (o & QSF_OUT_EPOT) != 0);
+    p.vtab = ob.pot_axis[0];
     p.kin_w = g.kinw.as<double>();
     p.dV = g.dV;
     p.dVm = g.dVm;
@@ -1824,7 +1873,7 @@ struct Prop {
     const bool flux = (o & QSF_OUT_FLUX) && pd.nborders > 0;
     const bool steers = pd.mode == QSF_MODE_IM && (o & QSF_OUT_EDIFF);
     if (o) p.flags |= LINE_OBS;
-    if (o & QSF_OUT_EPOT) p.flags |= LINE_EPOT;
+    if ((o & QSF_OUT_EPOT) && p.vtab) p.flags |= LINE_EPOT;   // (no potential: its sum is 0)
     if (ekin) p.flags |= LINE_EKIN;
     if (o & QSF_OUT_NORMALIZE) p.flags |= LINE_NORMALIZE;
     if (flux) {

@@ -30,7 +30,8 @@ def test_rows_together_and_one_at_a_time(case):
     borders = [(T.BORDER_BOX, box)] if box else [(b, 0) for b in T.ZOA_FLUX_2D]
     d = T.grid_desc(dim, n, 0.3, precision=prec, potential=T.POT_EBERLY, Ncharge=2, Echarge=-1, Nsoft=0.5, Esoft=0.33,
                     absorber=T.ABS_CAP, nCAP=8, multigrid=multi)
-    pd = T.prop_desc(T.MODE_RE, order, 0.02, gauge=gauge, outputs=T.OUT_NORM | T.OUT_EPOT | T.OUT_FLUX, borders=borders)
+    pd = T.prop_desc(T.MODE_RE, order, 0.02, gauge=gauge, outputs=T.OUT_NORM | T.OUT_EPOT | T.OUT_EKIN | T.OUT_FLUX,
+                     borders=borders)
     f = [T.field_desc([0, T.AXIS_X, T.AXIS_XY, T.AXIS_XYZ][dim], 0.1, 0.3, 2)]
     rng = np.random.default_rng(7)
     psi = (rng.normal(size=n ** dim) + 1j * rng.normal(size=n ** dim)) * 0.01
