@@ -102,6 +102,31 @@ __global__ void rows_flux_finish_kernel(RowSlots r, int blocks) {
   if (threadIdx.x == 0) r.rec[(int64_t)blockIdx.y * r.rec_width + 3 + b] = red[0] * r.flux.scale;
 }
 
+struct ProductBatch {
+  TableProduct p[16];
+};
+__global__ void table_products_kernel(ProductBatch b) {
+  const TableProduct& p = b.p[blockIdx.y];
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= p.n) return;
+  double2 z{1.0, 0.0};
+  for (int k = 0; k < p.count; ++k) z = cmul(z, p.in[k][i]);
+  p.out[i] = z;
+}
+
+void launch_table_products(const TableProduct* p, int count, hipStream_t s) {
+  for (int off = 0; off < count; off += 16) {
+    ProductBatch b{};
+    const int k = count - off < 16 ? count - off : 16;
+    int64_t nmax = 0;
+    for (int i = 0; i < k; ++i) {
+      b.p[i] = p[off + i];
+      nmax = p[off + i].n > nmax ? p[off + i].n : nmax;
+    }
+    hipLaunchKernelGGL(table_products_kernel, dim3((unsigned)((nmax + 255) / 256), (unsigned)k), dim3(256), 0, s, b);
+  }
+}
+
 int flux_blocks(int64_t npts) {
   const int64_t want = (npts + 255) / 256;
   return (int)(want < 1 ? 1 : (want > 1024 ? 1024 : want));

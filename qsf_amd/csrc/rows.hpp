@@ -19,6 +19,16 @@ struct RowSlots {
   int64_t nvals;
   double C[kRowSlots][3];    // velocity-gauge correction of each boundary
 };
+// out[i] = product of up to kFactors tables of n entries.
+struct TableProduct {
+  static constexpr int kFactors = 19;
+  double2* out;
+  int64_t n;
+  int32_t count;
+  const double2* in[kFactors];
+};
+void launch_table_products(const TableProduct* p, int count, hipStream_t s);
+
 int flux_blocks(int64_t npts);
 void launch_rows(int precision, const RowSlots& a, int slots, hipStream_t s);
 

@@ -1392,15 +1392,40 @@ struct Prop {
       }
       const SubOp& xl = ops.back();
       q.last[r] = g.x_factor(pd.mode, xl.delta, xl.C, couples() == QSF_REP_X);
+      if (whole_step_factor(g)) q.last[r] = step_product(g, q.subs[r], q.last[r]);
     }
     return q;
+  }
+
+  // A region with no transformed axis (XY of a plane) only multiplies: every factor of a step is a
+  // product of per-axis tables, so the step is one such product, left pending for the transfer
+  // that reads the region next. No pass of its own (two of 64 us a step at 2048^2 FP64, order 2).
+  bool whole_step_factor(const Grid& g) const {
+    return g.fftAxes.empty() && !g.pair_mask() && 2 * (int)chains.size() + 1 <= TableProduct::kFactors;
+  }
+  std::vector<TableProduct> products;
+  XFactor step_product(Grid& g, const std::vector<Sub>& subs, const XFactor& last) {
+    void* out = g.next_slot();
+    XFactor f{};
+    for (int a = 0; a < g.D; ++a) {
+      TableProduct t{};
+      t.n = g.n[a];
+      t.out = static_cast<double2*>(g.slot_axis(out, a));
+      for (const Sub& sb : subs)
+        for (const void* p : {sb.fb.axis[a], sb.pf[a]})
+          if (p) t.in[t.count++] = static_cast<const double2*>(p);
+      if (last.axis[a]) t.in[t.count++] = static_cast<const double2*>(last.axis[a]);
+      f.axis[a] = t.out;
+      products.push_back(t);
+    }
+    return f;
   }
 
   // Steps whose tables are built by one launch: as many as the ring of slots holds beside the
   // pending factor of the step before them.
   int64_t plan_ahead() const {
     const int K = (int)chains.size();
-    const int per = couples() == QSF_REP_X ? 2 * K + 1 : K;
+    const int per = (couples() == QSF_REP_X ? 2 * K + 1 : K) + (set->multi ? 1 : 0);
     return std::max(1, std::min(16, (Grid::kSlots - 2) / per - 1));
   }
 
@@ -1410,6 +1435,8 @@ struct Prop {
       std::vector<Plan> plans;
       for (int64_t k = 0; k < n; ++k) plans.push_back(plan_step());
       set->build_tables();
+      if (!products.empty()) launch_table_products(products.data(), (int)products.size(), st());
+      products.clear();
       for (const Plan& q : plans) {
         exec_fused(q);
         if (pd.outputs) request_row(q);
@@ -1421,25 +1448,36 @@ struct Prop {
   }
 
   void exec_fused(const Plan& plan) {
-    const std::vector<SubOp>& ops = plan.ops;
-    const size_t R = set->g.size();
-    for (size_t r = 0; r < R; ++r) {
-      Grid& g = *set->g[r];
-      if (r == 1 && pend_post) run_receives();
-      const bool obs_here = (r == 0) && pend_obs;
-      size_t k = 0;
-      for (size_t SI = 0; SI < ops.size(); ++SI) {
-        if (ops[SI].rep != QSF_REP_P) continue;
-        const bool first = (SI == 1);
-        const Sub& sb = plan.subs[r][k++];
-        run_p_substep(g, r, sb.fb, sb.pf, first && obs_here, first && r == 0 && pend_post);
-      }
-      pend[r].on = true;
-      pend[r].f = plan.last[r];
-      deferred[r] = true;
-    }
-    if (pend_obs) pend_obs = false;
+    main_step(plan);
+    if (pend_post) run_receives();
+    for (size_t r = 1; r < set->g.size(); ++r) region_step(r, plan);
+    pend_obs = false;
     if (set->multi) pend_post = true;
+  }
+
+  void main_step(const Plan& plan) {
+    Grid& g = main();
+    for (size_t k = 0; k < plan.subs[0].size(); ++k) {
+      const Sub& sb = plan.subs[0][k];
+      run_p_substep(g, 0, sb.fb, sb.pf, k == 0 && pend_obs, k == 0 && pend_post);
+    }
+    pend[0].on = true;
+    pend[0].f = plan.last[0];
+    deferred[0] = true;
+  }
+
+  // Region r >= 1: its substeps after its transfer.
+  void region_step(size_t r, const Plan& plan) {
+    Grid& g = *set->g[r];
+    if (whole_step_factor(g)) {
+      // (the transfers of the step before applied what was pending)
+      QSF_REQUIRE(!pend[r].on, QSF_ERR_STATE, "a region's factor is pending at the start of its step");
+    } else {
+      run_one_axis(g, r, plan.subs[r]);
+    }
+    pend[r].on = true;
+    pend[r].f = plan.last[r];
+    deferred[r] = true;
   }
 
   bool fused_multi() const { return set->multi && set->D == 2; }
@@ -1559,34 +1597,31 @@ struct Prop {
     }
   }
 
+  // Every P substep of a grid with one transformed axis: up to 1 + kMoreSubs of them in one pass, the
+  // state in registers between them (regions X and Y at 2048^2 FP64, order 2: two passes of 50 and
+  // 64 us become one).
+  void run_one_axis(Grid& g, size_t r, const std::vector<Sub>& subs) {
+    for (size_t k = 0; k < subs.size();) {
+      PassParams p = g.params(g.fftAxes[0], g.psi.p, g.psi.p);
+      p.flags = F_XB | F_FWD | F_P | F_INV2;
+      p.xb = subs[k].fb;
+      if (deferred[r] && pend[r].on) { p.flags |= F_XA; p.xa = pend[r].f; }
+      for (int a = 0; a < 3; ++a) p.pf[a] = subs[k].pf[a];
+      for (++k; k < subs.size() && p.nmore < kMoreSubs; ++k) {
+        MoreSub& m = p.more[p.nmore++];
+        m.x = subs[k].fb;
+        for (int a = 0; a < 3; ++a) m.pf[a] = subs[k].pf[a];
+      }
+      g.run(p);
+      deferred[r] = true;
+      pend[r].on = false;
+    }
+  }
+
   void run_p_substep(Grid& g, size_t r, const XFactor& fb, const void* const* pf, bool observe, bool post) {
     const int D = g.D;
     const auto& ax = g.fftAxes;
     const bool defer = deferred[r];
-    if (ax.empty()) {  // no transformed axis: pointwise pass
-      PassParams p = g.params(D - 1, g.psi.p, g.psi.p);
-      p.flags = F_XB | F_P;
-      p.xb = fb;
-      if (defer && pend[r].on) { p.flags |= F_XA; p.xa = pend[r].f; }
-      for (int a = 0; a < 3; ++a) p.pf[a] = pf[a];
-      g.run(p);
-      deferred[r] = true;
-      pend[r].on = false;
-      return;
-    }
-    if (ax.size() == 1) {  // one transformed axis: the whole substep is one pass
-      PassParams p = g.params(ax[0], g.psi.p, g.psi.p);
-      p.flags = F_XB | F_FWD | F_P | F_INV2;
-      p.xb = fb;
-      if (defer && pend[r].on) { p.flags |= F_XA; p.xa = pend[r].f; }
-      for (int a = 0; a < 3; ++a) p.pf[a] = pf[a];
-      if (observe) obs_into(g, p);
-      g.run(p);
-      if (observe) after_obs(g);
-      deferred[r] = true;
-      pend[r].on = false;
-      return;
-    }
     if (per_axis_kinetic(g)) {
       // 3D main grid: the kinetic factor is a product of commuting one-axis factors,
       // exp(-iT dt) = prod_d F_d^-1 f_d(p_d) F_d, so each axis pass transforms forward, applies
