@@ -127,6 +127,108 @@ void launch_table_products(const TableProduct* p, int count, hipStream_t s) {
   }
 }
 
+__global__ void ground_begin_kernel(double* state, int32_t* flags, double last_energy, int first) {
+  if (threadIdx.x) return;
+  if (first) state[0] = 1.0;
+  state[1] = last_energy;
+  flags[0] = flags[1] = 0;
+}
+
+// Four sums over [lo, hi) of the boundary pass' blocks followed by the kinetic passes' blocks:
+// norm, potential, kinetic of the boundary pass, kinetic of the others.
+__device__ __forceinline__ void ground_sums(const GroundRow& g, int64_t lo, int64_t hi, double* out) {
+  double a[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int64_t k = lo + threadIdx.x; k < hi; k += blockDim.x) {
+    if (k < g.tiles) {
+      for (int c = 0; c < 3; ++c) a[c] += g.sums[3 * k + c];
+    } else {
+      a[3] += g.kin[3 * (k - g.tiles) + 2];
+    }
+  }
+  __shared__ double red[4][16];
+  for (int c = 0; c < 4; ++c) {
+    for (int off = 32; off > 0; off >>= 1) a[c] += __shfl_xor(a[c], off);
+    if ((threadIdx.x & 63) == 0) red[c][threadIdx.x >> 6] = a[c];
+  }
+  block_sync();
+  for (int c = 0; c < 4; ++c) {
+    out[c] = 0.0;
+    for (int w = 0; w < (int)blockDim.x / 64; ++w) out[c] += red[c][w];
+  }
+}
+
+__global__ void __launch_bounds__(256) ground_chunks_kernel(GroundRow g, int64_t chunk) {
+  if (*g.flags) return;
+  const int64_t total = g.tiles + g.ktiles, lo = blockIdx.x * chunk, hi = lo + chunk < total ? lo + chunk : total;
+  double a[4];
+  ground_sums(g, lo, hi, a);
+  if (threadIdx.x < 4) g.scratch[4 * blockIdx.x + threadIdx.x] = a[threadIdx.x];
+}
+
+__global__ void __launch_bounds__(1024) ground_row_kernel(GroundRow g, int chunks) {
+  if (*g.flags) return;
+  double a[4];
+  if (chunks) {
+    // sums of the chunks, in order, by one thread per column
+    __shared__ double tot[4];
+    if (threadIdx.x < 4) {
+      double x = 0.0;
+#pragma unroll 8
+      for (int k = 0; k < chunks; ++k) x += g.scratch[4 * k + threadIdx.x];
+      tot[threadIdx.x] = x;
+    }
+    block_sync();
+    for (int c = 0; c < 4; ++c) a[c] = tot[c];
+  } else {
+    ground_sums(g, 0, g.tiles + g.ktiles, a);
+  }
+  if (threadIdx.x) return;
+  const double s = sqrt(1.0 / (a[0] * g.dV)), s2 = s * s;
+  const double epot = a[1] * s2, ekin = (a[2] + a[3]) * s2;
+  g.rec[0] = a[0] * s2;
+  g.rec[1] = epot;
+  g.rec[2] = ekin;
+  g.state[0] = s;
+  ++g.flags[1];
+  if (g.steers) {
+    // shouldContinue (propagator.h:304-309)
+    const double curr = __dadd_rn(__dmul_rn(epot, g.dV), __dmul_rn(ekin, g.dVm));
+    const double dif = curr - g.state[1];
+    g.state[1] = curr;
+    if (!(fabs(dif) > g.accuracy)) g.flags[0] = 1;
+  }
+}
+
+void launch_ground_begin(double* state, int32_t* flags, double last_energy, int first, hipStream_t s) {
+  hipLaunchKernelGGL(ground_begin_kernel, dim3(1), dim3(64), 0, s, state, flags, last_energy, first);
+}
+
+void launch_ground_row(const GroundRow& g, hipStream_t s) {
+  const int64_t total = g.tiles + g.ktiles;
+  if (total <= 8192) {
+    hipLaunchKernelGGL(ground_row_kernel, dim3(1), dim3(1024), 0, s, g, 0);
+    return;
+  }
+  hipLaunchKernelGGL(ground_chunks_kernel, dim3(256), dim3(256), 0, s, g, (total + 255) / 256);
+  hipLaunchKernelGGL(ground_row_kernel, dim3(1), dim3(64), 0, s, g, 256);
+}
+
+template <typename T> __global__ void ground_scale_kernel(T* psi, int64_t m, const double* state) {
+  const double sc = state[0];
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
+    const T v = psi[i];
+    psi[i] = T{(decltype(v.x))(v.x * sc), (decltype(v.x))(v.y * sc)};
+  }
+}
+
+void launch_ground_scale(int precision, void* psi, int64_t m, const double* state, hipStream_t s) {
+  const int blocks = (int)((m + 255) / 256 < 8192 ? (m + 255) / 256 : 8192);
+  if (precision == QSF_FP64)
+    hipLaunchKernelGGL(ground_scale_kernel<double2>, dim3(blocks), dim3(256), 0, s, (double2*)psi, m, state);
+  else
+    hipLaunchKernelGGL(ground_scale_kernel<float2>, dim3(blocks), dim3(256), 0, s, (float2*)psi, m, state);
+}
+
 int flux_blocks(int64_t npts) {
   const int64_t want = (npts + 255) / 256;
   return (int)(want < 1 ? 1 : (want > 1024 ? 1024 : want));

@@ -29,6 +29,25 @@ struct TableProduct {
 };
 void launch_table_products(const TableProduct* p, int count, hipStream_t s);
 
+// The row of one step boundary in imaginary time, from the block sums of the passes that read the
+// (not yet normalised) boundary state, and the scale that the next pass normalises it with.
+struct GroundRow {
+  const double* sums;        // [tiles][3]: norm, potential, kinetic sum of the last axis
+  int64_t tiles;
+  const double* kin;         // [ktiles][3]: kinetic sums of the other axes (third sum)
+  int64_t ktiles;
+  double* scratch;           // 256 * 4: second level (more than 8192 tiles)
+  double dV, dVm, accuracy;
+  int32_t steers;            // the energy difference ends the run (sets flags[0])
+  double* state;             // [0] scale, [1] energy of the row before
+  int32_t* flags;            // [0] halted, [1] rows taken
+  double* rec;               // norm, potential and kinetic sums of the normalised state
+};
+void launch_ground_begin(double* state, int32_t* flags, double last_energy, int first, hipStream_t s);
+void launch_ground_row(const GroundRow& g, hipStream_t s);
+// psi *= state[0] (the scale of the last row)
+void launch_ground_scale(int precision, void* psi, int64_t m, const double* state, hipStream_t s);
+
 int flux_blocks(int64_t npts);
 void launch_rows(int precision, const RowSlots& a, int slots, hipStream_t s);
 

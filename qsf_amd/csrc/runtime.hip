@@ -1885,11 +1885,10 @@ struct Prop {
       if (o & QSF_OUT_EPOT) row[3] = d[1] * g.dV;
       if (o & QSF_OUT_EKIN) row[4] = d[2] * g.dVm;
       if (o & QSF_OUT_ETOT) row[5] = d[1] * g.dV + d[2] * g.dVm;
-      if (o & QSF_OUT_EDIFF) {   // line runs only: the fused passes leave it to the member calls
-        const double curr = row[5] = d[1] * g.dV + d[2] * g.dVm;
+      if (o & QSF_OUT_EDIFF) {   // line runs and imaginary time
+        const double curr = d[1] * g.dV + d[2] * g.dVm;
         dif_energy = row[6] = curr - last_change;
         last_change = curr;
-        if (!(o & QSF_OUT_ETOT)) row[5] = std::nan("");
       }
       if (o & QSF_OUT_FLUX)
         for (int b = 0; b < pd.nborders; ++b) row[7 + b] = d[3 + b];
@@ -2061,6 +2060,140 @@ struct Prop {
     return done;
   }
 
+  // ---- imaginary time on planes and cubes: fused passes, normalisation on the device ----
+  // The member calls of a step sweep the state 25 (2D) to 37 (3D) times and wait for the host four
+  // times. Here the boundary pass forms the state, observes it and takes the last axis' kinetic
+  // sum from its registers; the other axes' sums are one read-only pass each; the scale that
+  // normalises the state is computed on the device and rides on the next step's first pass; and
+  // the energy difference halts the run by a flag that every later pass checks. 8 sweeps (2D).
+  bool ground_path() const {
+    if (!set || member_calls || pd.mode != QSF_MODE_IM || set->multi || set->D < 2) return false;
+    const int o = pd.outputs, both = QSF_OUT_EPOT | QSF_OUT_EKIN;
+    if (!(o & QSF_OUT_NORMALIZE) || fluxes() || radial_set()) return false;
+    return !(o & (QSF_OUT_ETOT | QSF_OUT_EDIFF)) || (o & both) == both;
+  }
+
+  DBuf ground_sums, ground_kin, ground_scratch, ground_state;
+
+  // Up to `want` steps (one chunk per host check of a steering energy difference); the state is
+  // normalised on return.
+  int64_t ground_steps(int64_t want) {
+    Grid& g = main();
+    const int D = g.D, o = pd.outputs;
+    const bool steers = o & QSF_OUT_EDIFF, ekin = o & (QSF_OUT_EKIN | QSF_OUT_ETOT);
+    const bool per_axis = per_axis_kinetic(g);
+    ground_scratch.ensure(256 * 4 * sizeof(double));
+    ground_state.ensure(2 * sizeof(double) + 2 * sizeof(int32_t));
+    double* gs = ground_state.as<double>();
+    int32_t* flags = reinterpret_cast<int32_t*>(gs + 2);
+    if (!devrec.p) {
+      devrec_cap = 4096;
+      devrec.ensure(devrec_cap * kRecWidth * sizeof(double));
+    }
+    int64_t taken = 0;
+    bool halted = false;
+    while (taken < want && !halted) {
+      if (devrec_used >= devrec_cap) sync_rows();
+      const int64_t n = std::min({want - taken, plan_ahead(), devrec_cap - devrec_used});
+      const phys::Coupling coup0 = coup;
+      const double timer0 = timer;
+      const int64_t step0 = step;
+      const size_t rows0 = rows.size(), pending0 = pending_rows.size();
+      std::vector<Plan> plans;
+      for (int64_t k = 0; k < n; ++k) {
+        plans.push_back(plan_step());
+        const std::vector<double> row = empty_row(plans.back().step, plans.back().timer);
+        pending_rows.push_back({(int)(rows.size() / width), ekin});
+        rows.insert(rows.end(), row.begin(), row.end());
+      }
+      set->build_tables();
+      launch_ground_begin(gs, flags, last_change, taken == 0, st());
+      for (int64_t k = 0; k < n; ++k) {
+        const Plan& q = plans[k];
+        for (size_t i = 0; i < q.subs[0].size(); ++i) {
+          const Sub& sb = q.subs[0][i];
+          for (int a = D - 1; a >= 0; --a) {
+            if (!per_axis && a > 0 && a < D - 1) continue;
+            PassParams p = g.params(a, g.psi.p, g.psi.p);
+            p.halt = flags;
+            if (a == D - 1) {
+              p.flags = F_XB | F_FWD;
+              p.xb = sb.fb;
+              if (i == 0) { p.flags |= F_SCALE; p.scale_dev = gs; }
+              else if (!per_axis) p.flags |= F_INV1;
+            }
+            if (per_axis) { p.flags |= F_FWD | F_P | F_INV2; p.pf[a] = sb.pf[a]; }
+            else if (a == 0) {
+              p.flags = F_FWD | F_P | F_INV2;
+              for (int b = 0; b < 3; ++b) p.pf[b] = sb.pf[b];
+            }
+            g.run(p);
+          }
+        }
+        GroundRow r{};
+        PassParams p = g.params(D - 1, g.psi.p, g.psi.p);
+        p.halt = flags;
+        p.flags = F_XA | F_OBS | F_KEEP | (per_axis ? 0u : F_INV1) | (ekin ? F_FWD | F_KIN : 0u);
+        p.xa = q.last[0];
+        g.obs_params(p.obs, (o & QSF_OUT_EPOT) != 0);
+        p.obs.kin_fwd = g.kin_axis(D - 1, false);
+        r.tiles = axis_pass_tiles(g.prec, p, g.variant(p));
+        ground_sums.ensure(r.tiles * 3 * sizeof(double));
+        p.obs.partials = ground_sums.as<double>();
+        g.run(p);
+        if (ekin) {
+          PassParams kp[2];
+          for (int a = 0; a < D - 1; ++a) {
+            kp[a] = g.kinetic_pass(a, g.psi.p);
+            r.ktiles += axis_pass_tiles(g.prec, kp[a], g.variant(kp[a]));
+          }
+          ground_kin.ensure(r.ktiles * 3 * sizeof(double));
+          double* out = ground_kin.as<double>();
+          for (int a = 0; a < D - 1; ++a) {
+            kp[a].halt = flags;
+            kp[a].obs.partials = out;
+            out += 3 * axis_pass_tiles(g.prec, kp[a], g.variant(kp[a]));
+            g.run(kp[a]);
+          }
+        }
+        r.sums = ground_sums.as<double>();
+        r.kin = ground_kin.as<double>();
+        r.scratch = ground_scratch.as<double>();
+        r.dV = g.dV;
+        r.dVm = g.dVm;
+        r.accuracy = state_accuracy;
+        r.steers = steers;
+        r.state = gs;
+        r.flags = flags;
+        r.rec = devrec.as<double>() + (size_t)(devrec_used + k) * kRecWidth;
+        launch_ground_row(r, st());
+        QSF_HIP(hipGetLastError());
+      }
+      int32_t fl[2] = {0, (int32_t)n};
+      if (steers) {
+        QSF_HIP(hipMemcpyAsync(fl, flags, sizeof(fl), hipMemcpyDeviceToHost, st()));
+        QSF_HIP(hipStreamSynchronize(st()));
+      }
+      halted = fl[0] != 0;
+      const int64_t done = fl[1];
+      devrec_used += done;
+      taken += done;
+      if (done < n) {
+        // the run halted early: the host side goes back to the steps that were taken
+        coup = coup0;
+        timer = timer0;
+        step = step0;
+        for (int64_t k = 0; k < done; ++k) schedule();
+        rows.resize(rows0 + (size_t)done * width);
+        pending_rows.resize(pending0 + done);
+      }
+      if (steers) sync_rows();   // the energy difference the loop is steered by
+    }
+    launch_ground_scale(g.prec, g.psi.p, g.m, gs, st());
+    QSF_HIP(hipGetLastError());
+    return taken;
+  }
+
   // the fused pipeline left work for the next pass (the grids are not at the step boundary), or
   // line runs since the last settle (their grid is at the boundary, and settling costs nothing)
   bool pending() const {
@@ -2113,6 +2246,10 @@ struct Prop {
   void loop_body() {
     if (line_path()) {
       line_steps(1);
+      return;
+    }
+    if (ground_path()) {
+      ground_steps(1);
       return;
     }
     if (fused()) {
@@ -2882,6 +3019,8 @@ int qsf_prop_run_steps(qsf_prop* p, int64_t k, int64_t* done) {
     while (i < k && p->p.should_continue()) {
       if (p->p.line_path()) {
         i += p->p.line_steps(std::min(k - i, p->p.steps_left()));
+      } else if (p->p.ground_path()) {
+        i += p->p.ground_steps(std::min(k - i, p->p.steps_left()));
       } else if (p->p.fused()) {
         const int64_t n = std::min(k - i, p->p.steps_left());
         p->p.run_fused(n);
