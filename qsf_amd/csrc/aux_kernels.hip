@@ -39,7 +39,7 @@ void launch_axis_tables(int precision, const AxisTableArgs* a, int count, hipStr
 template <typename Real>
 __global__ void pair_table_kernel(PairTableArgs a) {
   using T = typename cvec<Real>::T;
-  const int64_t total = a.kind == 1 ? a.n : a.n * a.n;
+  const int64_t total = a.kind == 1 ? a.n : a.n * a.n1;
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= total) return;
   double ee;
@@ -47,9 +47,10 @@ __global__ void pair_table_kernel(PairTableArgs a) {
     const double d = (double)k * a.dx;
     ee = a.EE / sqrt(d * d + a.Esoft);
   } else {
-    const int64_t i = k / a.n, j = k % a.n;
-    const double x = a.xmin + i * a.dx, y = a.xmin + j * a.dx;
-    if (a.model == QSF_POT_ECKHARDT_SACHA) ee = a.EE / sqrt((x - y) * (x - y) + x * y + a.Esoft);
+    const int64_t i = k / a.n1, j = k % a.n1;
+    const double x = a.xmin + i * a.dx, y = a.xmin1 + j * a.dx1;
+    if (a.model == QSF_POT_COULOMB) ee = a.NE / sqrt((x * x) + (y * y) + a.Nsoft);
+    else if (a.model == QSF_POT_ECKHARDT_SACHA) ee = a.EE / sqrt((x - y) * (x - y) + x * y + a.Esoft);
     else ee = a.EE / sqrt((x - y) * (x - y) + a.Esoft);
   }
   const double v = a.delta * ee;
@@ -116,7 +117,7 @@ void launch_radial_x(const RadialArgs& a, hipStream_t s) {
 }
 
 void launch_pair_table(int precision, const PairTableArgs& a, hipStream_t s) {
-  const int64_t total = a.kind == 1 ? a.n : a.n * a.n;
+  const int64_t total = a.kind == 1 ? a.n : a.n * a.n1;
   dim3 grid((unsigned)((total + 255) / 256));
   (void)precision;  // FP64 in both precisions (see launch_axis_tables)
   hipLaunchKernelGGL(pair_table_kernel<double>, grid, dim3(256), 0, s, a);

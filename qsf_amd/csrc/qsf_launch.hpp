@@ -58,10 +58,12 @@ struct AxisTableArgs {
 };
 void launch_axis_tables(int precision, const AxisTableArgs* a, int count, hipStream_t s);
 
-// Static pair tables exp(-iδ ee): kind PAIR_DIFF (n entries, |i-j|) or PAIR_FULL (n*n).
+// Static pair tables exp(-iδ ee): kind PAIR_DIFF (n entries, |i-j|) or PAIR_FULL (n*n1). Model
+// QSF_POT_COULOMB: the soft-core attraction over both coordinates (NE, Nsoft).
 struct PairTableArgs {
   void* out;
-  int64_t n;
+  int64_t n, n1;
+  double xmin1, dx1, NE, Nsoft;
   int32_t kind;          // PAIR_DIFF | PAIR_FULL
   int32_t model;         // QSF_POT_EBERLY | QSF_POT_ECKHARDT_SACHA
   int32_t mode;
