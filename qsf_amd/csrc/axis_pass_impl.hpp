@@ -760,6 +760,13 @@ constexpr bool tuned_length(int64_t n) {
   return n == 256 || n == 512 || n == 1024 || n == 2048 || n == 4096 || n == 768 || n == 1536;
 }
 inline bool has_variants(int64_t n) { return tuned_length(n); }
+// The one variant of every other length. In FP64 arithmetic the 3*2^k lengths from 48 on take the
+// 12-element plan (the 24-element one holds 210-250 registers, one or two waves per SIMD: 768-point
+// rows and columns, which have both, 26 -> 12 and 19 -> 13 us at 768^2); FP32 arithmetic keeps the
+// plan its results are rounded by.
+template <typename Real, int N> constexpr int default_variant() {
+  return !tuned_length(N) && sizeof(Real) == 8 && N % 3 == 0 && N >= 48 ? 3 : 0;
+}
 
 // Launcher and tile count of one axis length (all its variants). Instantiated explicitly per
 // (precision, mode, length group) in axis_pass_inst.hip, so the heavy kernels compile in
@@ -777,7 +784,7 @@ int launch_size(int v, const PassParams& p, hipStream_t s) {
       default: break;
     }
   }
-  return launch_one<Real, N, ROW, 0, S32>(p, s);
+  return launch_one<Real, N, ROW, default_variant<Real, N>(), S32>(p, s);
 }
 
 template <typename Real, bool ROW, int N>
@@ -792,7 +799,7 @@ int64_t tiles_size(int v, const PassParams& p) {
       default: break;
     }
   }
-  return tiles_one<Real, N, ROW, 0>(p);
+  return tiles_one<Real, N, ROW, default_variant<Real, N>()>(p);
 }
 
 #define QSF_SIZES(X) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048) X(4096) \
