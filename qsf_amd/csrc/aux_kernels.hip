@@ -648,41 +648,38 @@ void launch_batch_ptables(int precision, const BatchTableArgs* dev_args, int nso
 }
 
 // One block per solve: norm from the pass partials and the flux families from the gathered
-// boundary points, each a fixed-order sum (thread-strided, then a tree). The blocks are few (one
-// per solve of a size group) and the point loop is a chain of dependent loads, so the block is
-// as wide as it goes.
-constexpr int kObsThreads = 1024;
-template <typename Real>
+// boundary points. What bounds it is latency: a few blocks (one per solve of a size group) of a few
+// thousand values. Every sum is therefore kept in registers (families unrolled: indexed by a runtime
+// count they lived in scratch memory) and crosses the wave by shuffles and the block once for all of
+// them, two barriers in place of ten per family. Fixed order throughout.
+constexpr int kObsThreads = 1024, kObsFamilies = 16;
+template <typename Real, int D>
 __global__ void __launch_bounds__(kObsThreads)
     batch_obs_kernel(const BatchObsArgs* args, BatchFluxGeo geo, const int64_t* step_ctr) {
   using T = typename cvec<Real>::T;
   const BatchObsArgs& a = args[blockIdx.x];
   const int64_t k = *step_ctr;            // steps completed at the observed boundary
   if (k > a.total_steps || k < 1) return;
-  __shared__ double red[kObsThreads];
+  constexpr int NW = kObsThreads / 64;
+  __shared__ double red[kObsFamilies + 1][NW];
   double* row = a.rec + k * (1 + geo.nb);
   double acc = 0.0;
   for (int64_t b = threadIdx.x; b < a.tiles; b += kObsThreads) acc += a.partials[3 * b];
-  red[threadIdx.x] = acc;
-  block_sync();
-  for (int s = kObsThreads / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    block_sync();
-  }
-  if (threadIdx.x == 0) row[0] = red[0] * a.dV;
-  block_sync();
   const double* C = a.coupling + 3 * (k - 1);   // A after the step's P substep
   const T* g = reinterpret_cast<const T*>(a.gathered);
-  const int D = geo.D, nb = geo.nb, stride = 1 + 2 * D;
+  const int nb = geo.nb;
+  constexpr int stride = 1 + 2 * D;
   // one sweep over the points: each point's stencil is read once and its current added to every
   // family's sum (each family keeps its own per-thread order over the points)
-  double fam[16];
-  for (int f = 0; f < nb; ++f) fam[f] = 0.0;
+  double fam[kObsFamilies];
+#pragma unroll
+  for (int f = 0; f < kObsFamilies; ++f) fam[f] = 0.0;
   for (int64_t pidx = threadIdx.x; pidx < geo.npts; pidx += kObsThreads) {
     const int32_t* q = geo.pts + pidx * stride;
     const T c = g[q[0]];
     const double cr = c.x, ci = c.y, nrm = cr * cr + ci * ci;
-    double jd[3];
+    double jd[D];
+#pragma unroll
     for (int d = 0; d < D; ++d) {
       jd[d] = 0.0;
       const int32_t sp = q[1 + d], sm = q[1 + D + d];
@@ -692,37 +689,51 @@ __global__ void __launch_bounds__(kObsThreads)
       }
       jd[d] += C[d] * nrm;
     }
-    for (int f = 0; f < nb; ++f) {
+    const double* bv = geo.bvec + pidx * nb * D;
+#pragma unroll
+    for (int f = 0; f < kObsFamilies; ++f) {
+      if (f >= nb) break;
       double j = 0.0;
-      for (int d = 0; d < D; ++d) {
-        const double bv = geo.bvec[(pidx * nb + f) * D + d];
-        if (bv == 0.0) continue;
-        j += jd[d] * bv;
-      }
+#pragma unroll
+      for (int d = 0; d < D; ++d) j += jd[d] * bv[f * D + d];
       fam[f] += j;
     }
   }
-  for (int f = 0; f < nb; ++f) {
-    red[threadIdx.x] = fam[f];
-    block_sync();
-    for (int t = kObsThreads / 2; t > 0; t >>= 1) {
-      if ((int)threadIdx.x < t) red[threadIdx.x] += red[threadIdx.x + t];
-      block_sync();
-    }
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+  if (lane == 0) red[kObsFamilies][wave] = acc;
+#pragma unroll
+  for (int f = 0; f < kObsFamilies; ++f) {
+    if (f >= nb) break;
+    for (int off = 32; off > 0; off >>= 1) fam[f] += __shfl_xor(fam[f], off);
+    if (lane == 0) red[f][wave] = fam[f];
+  }
+  block_sync();
+  if (threadIdx.x <= nb) {
+    // thread 0: the norm; thread 1 + f: family f
+    const int f = threadIdx.x == 0 ? kObsFamilies : threadIdx.x - 1;
+    double x = 0.0;
+    for (int w = 0; w < NW; ++w) x += red[f][w];
     if (threadIdx.x == 0) {
-      row[1 + f] = red[0] * geo.scale;
+      row[0] = x * a.dV;
+    } else {
+      row[1 + f] = x * geo.scale;
       a.flux_int[f] += row[1 + f] * geo.dt;
     }
-    block_sync();
   }
 }
 
 void launch_batch_obs(const BatchObsArgs* dev_args, int nsolves, const BatchFluxGeo& geo,
                       const int64_t* step_ctr, hipStream_t s) {
-  if (geo.precision == QSF_FP64)
-    hipLaunchKernelGGL(batch_obs_kernel<double>, dim3(nsolves), dim3(kObsThreads), 0, s, dev_args, geo, step_ctr);
-  else
-    hipLaunchKernelGGL(batch_obs_kernel<float>, dim3(nsolves), dim3(kObsThreads), 0, s, dev_args, geo, step_ctr);
+  const dim3 grid(nsolves), block(kObsThreads);
+  const bool f64 = geo.precision == QSF_FP64;
+  if (geo.D == 1) {
+    if (f64) hipLaunchKernelGGL((batch_obs_kernel<double, 1>), grid, block, 0, s, dev_args, geo, step_ctr);
+    else hipLaunchKernelGGL((batch_obs_kernel<float, 1>), grid, block, 0, s, dev_args, geo, step_ctr);
+  } else {
+    if (f64) hipLaunchKernelGGL((batch_obs_kernel<double, 2>), grid, block, 0, s, dev_args, geo, step_ctr);
+    else hipLaunchKernelGGL((batch_obs_kernel<float, 2>), grid, block, 0, s, dev_args, geo, step_ctr);
+  }
 }
 
 __global__ void step_increment_kernel(int64_t* c) {
