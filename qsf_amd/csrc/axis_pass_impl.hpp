@@ -54,7 +54,8 @@ template <typename T, bool WAVE = false> struct RowAddr {
 template <typename T, int N> constexpr int row_stride() { return N + (N >> RowAddr<T>::SH); }
 
 // Kernel variant V (0..5): ALT = V / 3 selects the elements-per-thread plan, V % 3 scales the
-// tile width W (x1, x1/2, x2) within the LDS and block-size limits.
+// tile width W (x1, x1/2, x2) within the LDS and block-size limits. V = 6 is the mixed plan (ALT 2)
+// of the 5*2^k lengths in FP64 arithmetic.
 constexpr int kVariants = 6;
 constexpr int var_alt(int v) { return v / 3; }
 constexpr int var_wshift(int v) { return v % 3 == 0 ? 0 : (v % 3 == 1 ? -1 : 1); }
@@ -93,6 +94,11 @@ template <typename Real, int N, bool ROW, int V = 0> struct Geo {
   // the data the tile holds, which the occupancy budgets below are stated for
   static constexpr int lds_data(int w) { return w * N * CB; }
   static constexpr int base() {
+    if (PL::MIXED) {
+      // N/8 = 5*2^k threads a line: whole waves where a block takes 320 threads (40 KiB of LDS,
+      // three blocks or 15 waves a CU)
+      return T < 320 ? 320 / T : 1;
+    }
     if (ROW) {
       // at least 128 threads per block, at most 32 KiB of LDS: several blocks per CU overlap
       // their load, transform and store phases
@@ -327,7 +333,7 @@ __device__ __forceinline__ int64_t tile_at(const PassParams& p, int64_t k, int64
 // store. An observation leaves each wave's sums in the reduction area of LDS.
 template <typename Real, int N, bool ROW, int V, int FEAT, bool S32>
 __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, ROW, Geo<Real, N, ROW, V>::W>& g,
-                                          typename Tr<Real>::T (&v)[PlanOf<N, var_alt(V)>::E], int tid, int t, int w,
+                                          typename Tr<Real>::T (&v)[PlanOf<N, var_alt(V)>::SLOTS], int tid, int t, int w,
                                           unsigned char* smem_raw, StateOf<Real, S32>* dst, const void* pf0,
                                           const void* pf1, const void* pf2, void* gather_out) {
   using T = typename Tr<Real>::T;
@@ -335,7 +341,7 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
   using G = Geo<Real, N, ROW, V>;
   constexpr int ALT = var_alt(V);
   using PL = PlanOf<N, ALT>;
-  constexpr int E = PL::E, TT = PL::T;
+  constexpr int E = PL::E, SLOTS = PL::SLOTS, TT = PL::T;
   constexpr int W = Geo<Real, N, ROW, V>::W;
   T* lds = reinterpret_cast<T*>(smem_raw);
   T* glds = reinterpret_cast<T*>(smem_raw + G::gather_off);
@@ -360,7 +366,7 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
     // with one rounding; a once-rounded FP32 scale would bias the norm the same way every step
     const double sc = p.scale_dev ? p.scale * *p.scale_dev : p.scale;
 #pragma unroll
-    for (int q = 0; q < E; ++q) v[q] = capply(v[q], double2{sc, 0.0});
+    for (int q = 0; q < SLOTS; ++q) v[q] = capply(v[q], double2{sc, 0.0});
   }
 
   int tx = t;
@@ -385,8 +391,9 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
     double ek = 0.0;
     if (valid) {
 #pragma unroll
-      for (int q = 0; q < E; ++q)
-        ek += ((double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y) * kw[t + TT * q];
+      for (int q = 0; q < SLOTS; ++q)
+        if (PL::xhas(t, q))
+          ek += ((double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y) * kw[PL::xpos(t, q)];
     }
     for (int off = 32; off > 0; off >>= 1) ek += __shfl_xor(ek, off);
     double* red = reinterpret_cast<double*>(smem_raw + G::red_off);
@@ -448,8 +455,9 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
                          (FEAT == FEAT_BOUNDARY && !keep && !(obs && ob.copy_out));
     if (compact) {
 #pragma unroll
-      for (int q = 0; q < E; ++q) {
-        const int ia = t + TT * q;
+      for (int q = 0; q < SLOTS; ++q) {
+        const int ia = PL::xpos(t, q);
+        const bool has = PL::xhas(t, q);
         double2 zab{1.0, 0.0};
         double wa = 1.0;   // |A factor|^2
         if (same) {
@@ -467,7 +475,7 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
         } else if (doB) {
           zab = xb.at(ia);
         }
-        if (obs && valid) {
+        if (obs && valid && has) {
           const double a2 = ((double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y) * wa;
           nrm += a2;
           if constexpr (FEAT == FEAT_BOUNDARY) {
@@ -475,30 +483,31 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
           }
           if (ka || kc != 0.0) ek += a2 * (kc + (ka ? ka[ia] : 0.0));
         }
-        if (gline) glds[w * G::gather_stride + ia] = v[q];
+        if (gline && has) glds[w * G::gather_stride + ia] = v[q];
         if (doA || doB) v[q] = capply(v[q], zab);
       }
     } else if constexpr (FEAT == FEAT_BOUNDARY || FEAT == FEAT_FULL) {
 #pragma unroll
-    for (int q = 0; q < E; ++q) {
-      const int ia = t + TT * q;
+    for (int q = 0; q < SLOTS; ++q) {
+      const int ia = PL::xpos(t, q);
+      const bool has = PL::xhas(t, q);
       double2 pp, za;
       if (shared) pp = xa.pair_at(ia);
       if (doA) {
         za = shared ? cmul(xa.base_at(ia), pp) : xa.at(ia);
         v[q] = capply(v[q], za);
       }
-      if (obs && valid) {
+      if (obs && valid && has) {
         const double a2 = (double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y;
         nrm += a2;
         if (ob.want_epot) ep += a2 * pot.at(ob, p.axis, ia);
         if (ka || kc != 0.0) ek += a2 * (kc + (ka ? ka[ia] : 0.0));
         if (ob.copy_out) reinterpret_cast<S*>(ob.copy_out)[base + (int64_t)ia * step] = to_state<S>(v[q]);
       }
-      if (keep && valid) dst[base + (int64_t)ia * step] = to_state<S>(v[q]);
-      if (gline) glds[w * G::gather_stride + ia] = v[q];
+      if (keep && valid && has) dst[base + (int64_t)ia * step] = to_state<S>(v[q]);
+      if (gline && has) glds[w * G::gather_stride + ia] = v[q];
       if constexpr (FEAT == FEAT_FULL) {
-      if (ROW && p.er_out && valid) {
+      if (ROW && p.er_out && valid && has) {
         // multigrid source edges of the boundary state (2D main region, row i0 = o)
         const int64_t nc = p.nCAP, n0 = p.n[0], n1 = N;
         if (o < nc || o >= n0 - nc) {
@@ -563,12 +572,12 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
       if (sub > 0) {
         if constexpr (!std::is_same_v<S, T>) {
 #pragma unroll
-          for (int q = 0; q < E; ++q) v[q] = from_state<T>(to_state<S>(v[q]));   // rounded as a pass stores it
+          for (int q = 0; q < SLOTS; ++q) v[q] = from_state<T>(to_state<S>(v[q]));   // rounded as a pass stores it
         }
         XEval<N> x;
         x.init(p.more[sub - 1].x, p.axis, i0, i1, i2);
 #pragma unroll
-        for (int q = 0; q < E; ++q) v[q] = capply(v[q], x.at(t + TT * q));
+        for (int q = 0; q < SLOTS; ++q) v[q] = capply(v[q], x.at(PL::xpos(t, q)));
       }
     }
     if (p.flags & F_FWD) run_fft(FWD{});
@@ -598,10 +607,15 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
       if (p.axis != 1 && f1) cst = cmul(cst, ld<double2>(f1, i1));
       if (p.axis != 2 && f2) cst = cmul(cst, ld<double2>(f2, i2));
       const double2* pa = reinterpret_cast<const double2*>(p.axis == 0 ? f0 : (p.axis == 1 ? f1 : f2));
+      if (!PL::MIXED || (p.flags & F_FWD)) {
 #pragma unroll
-      for (int q = 0; q < E; ++q) {
-        const double2 f = pa ? cmul(cst, pa[t + TT * q]) : cst;
-        v[q] = capply(v[q], f);
+        for (int q = 0; q < E; ++q) {
+          const double2 f = pa ? cmul(cst, pa[t + TT * q]) : cst;
+          v[q] = capply(v[q], f);
+        }
+      } else {   // a P factor beside no transform: the slots the state was loaded into
+#pragma unroll
+        for (int q = 0; q < SLOTS; ++q) v[q] = capply(v[q], pa ? cmul(cst, pa[PL::xpos(t, q)]) : cst);
       }
     }
 
@@ -610,6 +624,14 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
   }
 
   if (valid && !(p.flags & (F_NOSTORE | F_KEEP))) {
+    if constexpr (PL::MIXED) {
+      if (!(p.flags & F_FWD) || (p.flags & F_INV2)) {   // the X side, in the first stage's slots
+#pragma unroll
+        for (int q = 0; q < SLOTS; ++q)
+          if (PL::xhas(t, q)) dst[base + (int64_t)PL::xpos(t, q) * step] = to_state<S>(v[q]);
+        return;
+      }
+    }
 #pragma unroll
     for (int q = 0; q < E; ++q) dst[base + (int64_t)(t + TT * q) * step] = to_state<S>(v[q]);
   }
@@ -640,7 +662,7 @@ __global__ void __launch_bounds__((Geo<Real, N, ROW, V>::THREADS),
   using T = typename Tr<Real>::T;
   constexpr int ALT = var_alt(V);
   using PL = PlanOf<N, ALT>;
-  constexpr int E = PL::E, TT = PL::T;
+  constexpr int E = PL::E, SLOTS = PL::SLOTS, TT = PL::T;
   constexpr int W = Geo<Real, N, ROW, V>::W;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   if (p.halt && *p.halt) return;   // (the whole grid: the flag changes only between passes)
@@ -680,10 +702,18 @@ __global__ void __launch_bounds__((Geo<Real, N, ROW, V>::THREADS),
   const int64_t k0 = (nb & 7) == 0 ? (int64_t)(blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3) : (int64_t)blockIdx.x;
   TileGeo<N, ROW, W> g;
   g.at(p, tile_at<W, ROW>(p, k0, ntiles), w);
-  T v[E];
+  T v[SLOTS];
+  if (PL::MIXED && !(p.flags & F_INV1)) {   // (an inverse alone is an F_INV1: F_INV2 follows F_FWD)
 #pragma unroll
-  for (int q = 0; q < E; ++q)
-    v[q] = g.valid ? from_state<T>(src[g.base + (int64_t)(t + TT * q) * g.step]) : T{Real(0), Real(0)};
+    for (int q = 0; q < SLOTS; ++q)
+      v[q] = g.valid && PL::xhas(t, q) ? from_state<T>(src[g.base + (int64_t)PL::xpos(t, q) * g.step]) : T{Real(0), Real(0)};
+  } else {
+#pragma unroll
+    for (int q = 0; q < E; ++q)
+      v[q] = g.valid ? from_state<T>(src[g.base + (int64_t)(t + TT * q) * g.step]) : T{Real(0), Real(0)};
+#pragma unroll
+    for (int q = E; q < SLOTS; ++q) v[q] = T{Real(0), Real(0)};
+  }
   pass_tile<Real, N, ROW, V, FEAT, S32>(p, g, v, tid, t, w, smem_raw, dst, pf0, pf1, pf2, gather_out);
   if (FEAT != FEAT_LEAN && (p.flags & F_OBS)) {
     // the block's sums: its waves' sums in wave order
@@ -765,6 +795,7 @@ inline bool has_variants(int64_t n) { return tuned_length(n); }
 // rows and columns, which have both, 26 -> 12 and 19 -> 13 us at 768^2); FP32 arithmetic keeps the
 // plan its results are rounded by.
 template <typename Real, int N> constexpr int default_variant() {
+  if (sizeof(Real) == 8 && N % 5 == 0 && N >= 80) return 6;
   return !tuned_length(N) && sizeof(Real) == 8 && N % 3 == 0 && N >= 48 ? 3 : 0;
 }
 

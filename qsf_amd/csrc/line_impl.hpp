@@ -15,17 +15,17 @@
 // stay in registers, or in LDS where the plan needs more than six records. Measured, a step: 4096
 // points FP64, length gauge, energies and flux 49.9 -> 11.1 us (seven single-block launches before);
 // 1536 points FP32, norm and flux 29.6 -> 10.9 us; 2560 points FP64 in imaginary time, with its
-// four host round trips gone, 197 -> 25.5 us.
+// four host round trips gone, 197 -> 25.5 us, by the mixed plan (five waves in place of two) 14.7 us.
 #include "axis_pass_impl.hpp"
 
 namespace qsf {
 
 // Plan of a line in FP64 arithmetic: eight elements per thread where the length allows it (twelve
-// for 3*2^k, twenty for 5*2^k), so the long lines spread over all four SIMDs of the CU. FP32
+// for 3*2^k; the mixed plan for 5*2^k), so the long lines spread over all four SIMDs of the CU. FP32
 // arithmetic keeps the plan of the tuned axis pass instead (each factorisation rounds its own way,
 // and an FP32 run then gives the values it gives through the passes, whatever the path).
 constexpr int line_alt(int n) {
-  if (n % 5 == 0) return 0;
+  if (n % 5 == 0) return n >= 80 ? 2 : 0;
   if (n % 3 == 0) return n >= 48 ? 1 : 0;
   return n >= 128 && n != 512 ? 1 : 0;
 }
@@ -48,8 +48,9 @@ template <typename Real, int N, int LALT> struct LineGeo {
   using PL = PlanOf<N, ALT>;
   static constexpr int TT = PL::T;
   // lines shorter than a wave's 64 threads are held several times over (only copy 0 is stored and
-  // counted), so every lane of the wave takes part in the sums
-  static constexpr int THREADS = TT < 64 ? 64 : TT;
+  // counted), so every lane of the wave takes part in the sums; where the line's threads are no whole
+  // number of waves (the mixed plan) the lanes left over repeat its first threads, in the same LDS image
+  static constexpr int THREADS = (TT + 63) / 64 * 64;
   static constexpr int COPIES = THREADS / TT;
   static constexpr int NWAVES = THREADS / 64;
   static constexpr bool WAVE = TT <= 64;
@@ -66,7 +67,8 @@ __global__ void __launch_bounds__((LineGeo<Real, N, LALT>::THREADS)) line_kernel
   using G = LineGeo<Real, N, LALT>;
   using T = typename Tr<Real>::T;
   using S = StateOf<Real, S32>;
-  constexpr int ALT = G::ALT, E = G::PL::E, TT = G::TT;
+  using PL = typename G::PL;
+  constexpr int ALT = G::ALT, E = PL::E, SLOTS = PL::SLOTS, TT = G::TT;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T* lds = reinterpret_cast<T*>(smem_raw);
   double* red = reinterpret_cast<double*>(smem_raw + G::red_off);
@@ -74,9 +76,9 @@ __global__ void __launch_bounds__((LineGeo<Real, N, LALT>::THREADS)) line_kernel
   const bool valid = copy == 0;
   S* psi = reinterpret_cast<S*>(p.psi);
 
-  T v[E];
+  T v[SLOTS];
 #pragma unroll
-  for (int q = 0; q < E; ++q) v[q] = from_state<T>(psi[t + TT * q]);
+  for (int q = 0; q < SLOTS; ++q) v[q] = from_state<T>(psi[PL::xpos(t, q)]);
   const T* roots = reinterpret_cast<const T*>(p.roots);
   if constexpr (G::LDS_ROOTS) {
     float4* dst = reinterpret_cast<float4*>(smem_raw + G::roots_off);   // 16 bytes per root
@@ -87,21 +89,21 @@ __global__ void __launch_bounds__((LineGeo<Real, N, LALT>::THREADS)) line_kernel
   }
   Twiddles<N, ALT, T> tw;
   tw.load(roots, t);
-  LineAddr<T, G::STRIDE, G::WAVE> addr{G::WAVE ? copy * G::STRIDE : 0};
+  LineAddr<T, G::STRIDE, G::WAVE> addr{G::WAVE && !PL::MIXED ? copy * G::STRIDE : 0};
   // the flux stencil slots of this thread's nodes
   const bool epot = p.flags & LINE_EPOT, ekin = p.flags & LINE_EKIN, flux = p.flags & LINE_FLUX;
   const bool obs = p.flags & LINE_OBS, normalise = p.flags & LINE_NORMALIZE;
   const bool formed = ekin || normalise;   // the boundary state itself is needed
-  int slot[E];
+  int slot[SLOTS];
   bool any = false;
 #pragma unroll
-  for (int q = 0; q < E; ++q) slot[q] = -1;
+  for (int q = 0; q < SLOTS; ++q) slot[q] = -1;
   if (flux && valid)
     for (int k = 0; k < p.nvals; ++k) {
       const int pos = p.gather_pos[k];
 #pragma unroll
-      for (int q = 0; q < E; ++q)
-        if (t + TT * q == pos) { slot[q] = k; any = true; }
+      for (int q = 0; q < SLOTS; ++q)
+        if (PL::xhas(t, q) && PL::xpos(t, q) == pos) { slot[q] = k; any = true; }
     }
 
   // The step loop would otherwise hoist every power of the twiddles out of itself (84 registers at
@@ -139,11 +141,11 @@ __global__ void __launch_bounds__((LineGeo<Real, N, LALT>::THREADS)) line_kernel
     }
   };
 
-  double2 za[E];        // the trailing X factor of the last step, where it is still to be applied
+  double2 za[SLOTS];        // the trailing X factor of the last step, where it is still to be applied
   bool pend = p.za_in != nullptr;
   if (pend) {
 #pragma unroll
-    for (int q = 0; q < E; ++q) za[q] = p.za_in[t + TT * q];
+    for (int q = 0; q < SLOTS; ++q) za[q] = p.za_in[PL::xpos(t, q)];
   }
   double last = p.last_energy;
   int done = 0;
@@ -154,8 +156,8 @@ __global__ void __launch_bounds__((LineGeo<Real, N, LALT>::THREADS)) line_kernel
       {
         const double2* x = xt + (int64_t)sub * N;
 #pragma unroll
-        for (int q = 0; q < E; ++q) {
-          double2 z = x[t + TT * q];
+        for (int q = 0; q < SLOTS; ++q) {
+          double2 z = x[PL::xpos(t, q)];
           if (sub == 0 && pend) z = cmul(za[q], z);
           v[q] = capply(v[q], z);
         }
@@ -169,14 +171,14 @@ __global__ void __launch_bounds__((LineGeo<Real, N, LALT>::THREADS)) line_kernel
       for (int q = 0; q < E; ++q) v[q] = capply(v[q], f[q]);
       if (sub == p.nsub - 1) {
 #pragma unroll
-        for (int q = 0; q < E; ++q) za[q] = xt[(int64_t)p.nsub * N + t + TT * q];
+        for (int q = 0; q < SLOTS; ++q) za[q] = xt[(int64_t)p.nsub * N + t + (PL::xpos(t, q) - t)];
       }
       transform(v, INV{});
       if constexpr (S32) {
         // the FP32 state is rounded once a substep, as the passes store it: a run's result does
         // not depend on how its steps are split into launches
 #pragma unroll
-        for (int q = 0; q < E; ++q) v[q] = from_state<T>(to_state<S>(v[q]));
+        for (int q = 0; q < SLOTS; ++q) v[q] = from_state<T>(to_state<S>(v[q]));
       }
     }
     pend = true;
@@ -185,36 +187,38 @@ __global__ void __launch_bounds__((LineGeo<Real, N, LALT>::THREADS)) line_kernel
     // the step boundary: observables weight |psi|^2 by |A|^2 where the state is not formed
     if (formed) {
 #pragma unroll
-      for (int q = 0; q < E; ++q) v[q] = capply(v[q], za[q]);
+      for (int q = 0; q < SLOTS; ++q) v[q] = capply(v[q], za[q]);
       pend = false;
     }
     if (normalise) {
       double a = 0.0;
 #pragma unroll
-      for (int q = 0; q < E; ++q) a += (double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y;
+      for (int q = 0; q < SLOTS; ++q)
+        if (PL::xhas(t, q)) a += (double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y;
       const double nrm = block_sum(wave_sum(valid ? a : 0.0));
       const double sc = sqrt(1.0 / (nrm * p.dV));
 #pragma unroll
-      for (int q = 0; q < E; ++q) v[q] = T{(Real)((double)v[q].x * sc), (Real)((double)v[q].y * sc)};
+      for (int q = 0; q < SLOTS; ++q) v[q] = T{(Real)((double)v[q].x * sc), (Real)((double)v[q].y * sc)};
     }
     double nrm = 0.0, ep = 0.0, ek = 0.0;
 #pragma unroll
-    for (int q = 0; q < E; ++q) {
+    for (int q = 0; q < SLOTS; ++q) {
+      if (!PL::xhas(t, q)) continue;
       double a2 = (double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y;
       if (!formed) a2 *= cabs2(za[q]);
       nrm += a2;
-      if (epot) ep += a2 * p.vtab[t + TT * q];
+      if (epot) ep += a2 * p.vtab[PL::xpos(t, q)];
     }
     if (any) {
       T* go = reinterpret_cast<T*>(p.gathered) + (int64_t)s * p.nvals;
 #pragma unroll
-      for (int q = 0; q < E; ++q)
+      for (int q = 0; q < SLOTS; ++q)
         if (slot[q] >= 0) go[slot[q]] = formed ? v[q] : capply(v[q], za[q]);
     }
     if (ekin) {
-      T u[E];
+      T u[SLOTS];
 #pragma unroll
-      for (int q = 0; q < E; ++q) u[q] = v[q];
+      for (int q = 0; q < SLOTS; ++q) u[q] = v[q];
       transform(u, FWD{});
 #pragma unroll
       for (int q = 0; q < E; ++q)
@@ -240,7 +244,8 @@ __global__ void __launch_bounds__((LineGeo<Real, N, LALT>::THREADS)) line_kernel
   // a trailing factor that no observation formed stays pending: it meets the next run's first half
   if (valid) {
 #pragma unroll
-    for (int q = 0; q < E; ++q) psi[t + TT * q] = to_state<S>(v[q]);
+    for (int q = 0; q < SLOTS; ++q)
+      if (PL::xhas(t, q)) psi[PL::xpos(t, q)] = to_state<S>(v[q]);
   }
   if (tid == 0 && p.done) *p.done = done;
 }

@@ -6,6 +6,7 @@
   tiles, unequal sides, one and two substeps, with and without the kinetic energy, and a stop inside
   a run of steps.
 * CoulombInteraction over both coordinates of a plane with unequal sides (a table factor in FP64).
+* The mixed plan of the 5*2^k lengths at partial tiles.
 
 Bars as for the axis passes: psi 1e-10 FP64, 1e-4 FP32-mixed, 2e-6 FP32 state; records 1e-9 / 1e-4 /
 1e-5 of each column's largest value (fluxes in FP64 only, where they are a difference of
@@ -133,3 +134,17 @@ def test_coulomb_plane_with_unequal_sides(ctx, shape):
         got, want = both(ctx, shape, T.FP64, pd, f, (4, 1, 3), potential=T.POT_COULOMB, Ncharge=1, Echarge=-1, Nsoft=0.7,
                          absorber=T.ABS_CAP, nCAP=6)
         check(got, want, T.FP64)
+
+
+MIXED_SHAPES = [(80, 20), (20, 80), (160, 48), (24, 320), (320, 12), (640, 40), (1280, 10), (16, 1280), (2560, 8), (8, 2560)]
+
+
+@pytest.mark.parametrize("shape", MIXED_SHAPES, ids=["x".join(map(str, s)) for s in MIXED_SHAPES])
+def test_mixed_plan_partial_tiles(ctx, shape):
+    """The mixed plan of the 5*2^k lengths beside short axes: tiles with idle lines and columns."""
+    print(f"[case] mixed {shape}", flush=True)
+    f = [T.field_desc(T.AXIS_XY, 0.1, 0.3, 2)]
+    pd = T.prop_desc(T.MODE_RE, 1, 0.04, gauge=T.GAUGE_LENGTH, outputs=T.OUT_NORM | T.OUT_EPOT | T.OUT_EKIN)
+    for prec in (T.FP64, T.FP32_STATE):
+        got, want = both(ctx, shape, prec, pd, f, (3, 1), potential=T.POT_COULOMB, Ncharge=1, Echarge=-1, Nsoft=0.7)
+        check(got, want, prec)
