@@ -206,6 +206,13 @@ template <int N> struct XEval {
     if (npr > 1) r = cmul(r, kind == PAIR_DIFF ? pr1[abs(n - o1)] : pr1[n]);
     return r;
   }
+  // the same with their number known and without a branch: |n - off| indexes both kinds of table
+  __device__ __forceinline__ int off0() const { return kind == PAIR_DIFF ? o0 : 0; }
+  __device__ __forceinline__ int off1() const { return kind == PAIR_DIFF ? o1 : 0; }
+  template <int NPR> __device__ __forceinline__ T pairs(int n) const {
+    if constexpr (NPR == 1) return pr0[abs(n - off0())];
+    else return cmul(pr0[abs(n - off0())], pr1[abs(n - off1())]);
+  }
   // factor without the axis-dependent pair part
   __device__ __forceinline__ T base_at(int n) const { return ax ? cmul(cst, ax[n]) : cst; }
   __device__ __forceinline__ T at(int n) const { return npr ? cmul(base_at(n), pair_at(n)) : base_at(n); }
@@ -266,6 +273,11 @@ struct PotEval {
     }
     return v;
   }
+  template <int NPR> __device__ __forceinline__ double tables(int n) const {
+    double v = cst + ax[n] + pr0[abs(n - (kind == PAIR_DIFF ? o0 : 0))];
+    if constexpr (NPR > 1) v += pr1[abs(n - (kind == PAIR_DIFF ? o1 : 0))];
+    return v;
+  }
 };
 
 // Geometry of one thread's transform in tile b: (outer o, inner c), its global offsets and the
@@ -299,7 +311,9 @@ struct TileGeo {
       i0 = (int)(o / p.n[1]);
       i1 = (int)(o % p.n[1]);
     }
-    if (!valid) i0 = i1 = i2 = 0;   // idle threads of a partial tile read in-range table entries
+    // idle threads of a partial tile read in range (the first line and its table entries); none of
+    // their values is stored or counted
+    if (!valid) { base = 0; i0 = i1 = i2 = 0; }
   }
 };
 
@@ -453,7 +467,115 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
     const bool keep = p.flags & F_KEEP;
     const bool compact = FEAT == FEAT_X || FEAT == FEAT_MORE ||
                          (FEAT == FEAT_BOUNDARY && !keep && !(obs && ob.copy_out));
-    if (compact) {
+    // Usual forms of the stage, an interaction term along the line and both halves (or the formed
+    // state's one): everything that selects a form is decided before the loop over the elements, which
+    // then has no branch, so the table loads of a group of elements are issued together. With the
+    // selections inside, each element waited for its own loads (256^2 FP64 rows 10.3 -> 7.6 us, 768^2
+    // FP64 rows that keep the state 24.5 -> 17.7, 320^3 FP32 state rows 672 -> 569). A group's tables take about
+    // 40 registers (24 where a thread holds more than ten elements); without the fences between groups
+    // the scheduler issues every load of the line at once and spills 140 to 300 registers. The more and
+    // full tiers keep the loop below: they have no registers to spare (2048-point rows in groups: the
+    // more tier spilled 128, the full tier fell from three waves to two, the regions' step 12% slower).
+    constexpr int BUDGET = SLOTS <= 10 ? 40 : 24;
+    auto settled = [&](T& x) {
+      asm volatile("" : "+v"(x.x), "+v"(x.y), "+v"(nrm), "+v"(ep) : : "memory");
+    };
+    auto form = [&](auto npr_tag, auto same_tag) {
+      constexpr int NPR = decltype(npr_tag)::value;
+      constexpr bool SAME = decltype(same_tag)::value;
+      constexpr int GROUP = BUDGET / (4 * (1 + NPR + (SAME ? 0 : 1)));
+      if (gline) {
+#pragma unroll
+        for (int q = 0; q < SLOTS; ++q)
+          if (PL::xhas(t, q)) glds[w * G::gather_stride + PL::xpos(t, q)] = v[q];
+      }
+#pragma unroll
+      for (int q = 0; q < SLOTS; ++q) {
+        const int ia = PL::xpos(t, q);
+        double2 zab;
+        double wa;   // |A factor|^2
+        if constexpr (SAME) {
+          const double2 z = cmul(cmul(xa.cst, xa.ax[ia]), xa.template pairs<NPR>(ia));
+          zab = cmul(z, z);
+          wa = cabs2(z);
+        } else {
+          const double2 pp = xa.template pairs<NPR>(ia), ba = cmul(xa.cst, xa.ax[ia]);
+          zab = cmul(cmul(ba, cmul(xb.cst, xb.ax[ia])), cmul(pp, pp));
+          wa = cabs2(ba) * cabs2(pp);
+        }
+        const double a2 = ((double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y) * wa;
+        nrm += valid && PL::xhas(t, q) ? a2 : 0.0;
+        v[q] = capply(v[q], zab);
+        if (q % GROUP == GROUP - 1)
+          for (int r = q - GROUP + 1; r <= q; ++r) settled(v[r]);
+      }
+    };
+    // the state formed between the halves: copied, or kept in place of the pass's result (no second
+    // half then: B 0); B 1 repeats the first half, B 2 shares its interaction term
+    auto form_kept = [&](auto npr_tag, auto epot_tag, auto b_tag) {
+      constexpr int NPR = decltype(npr_tag)::value, B = decltype(b_tag)::value;
+      constexpr bool EPOT = decltype(epot_tag)::value;
+      constexpr int GROUP = std::max(1, BUDGET / (4 * (1 + NPR + (B == 2 ? 1 : 0)) + (EPOT ? 2 + 2 * NPR : 0)));
+      S* out = B == 0 ? dst : reinterpret_cast<S*>(ob.copy_out);
+#pragma unroll
+      for (int q0 = 0; q0 < SLOTS; q0 += GROUP) {
+        int t = tx;   // opaque: the addresses of a group are formed within it, not kept from another
+        asm volatile("" : "+v"(t));
+        double2 z[GROUP];
+#pragma unroll
+        for (int q = q0; q < q0 + GROUP && q < SLOTS; ++q) {
+          const int ia = PL::xpos(t, q);
+          const double2 pp = xa.template pairs<NPR>(ia), za = cmul(cmul(xa.cst, xa.ax[ia]), pp);
+          v[q] = capply(v[q], za);
+          z[q - q0] = B == 2 ? cmul(cmul(xb.cst, xb.ax[ia]), pp) : za;
+          const double a2 = (double)v[q].x * (double)v[q].x + (double)v[q].y * (double)v[q].y;
+          const double counted = valid && PL::xhas(t, q) ? a2 : 0.0;
+          nrm += counted;
+          if constexpr (EPOT) ep += counted * pot.template tables<NPR>(ia);
+        }
+#pragma unroll
+        for (int q = q0; q < q0 + GROUP && q < SLOTS; ++q) {
+          if (valid && PL::xhas(t, q)) {
+            out[base + (int64_t)PL::xpos(t, q) * step] = to_state<S>(v[q]);
+            if (gline) glds[w * G::gather_stride + PL::xpos(t, q)] = v[q];
+          }
+          if constexpr (B != 0) v[q] = capply(v[q], z[q - q0]);
+          settled(v[q]);
+        }
+      }
+    };
+    using std::integral_constant;
+    const bool bare = obs && !ka && kc == 0.0 && xa.ax;   // no weights but the potential's
+    bool kept = false;
+    if constexpr (FEAT == FEAT_BOUNDARY) {
+      using One = integral_constant<int, 1>;
+      using Two = integral_constant<int, 2>;
+      const bool epot = ob.want_epot, tabled = !epot || (pot.ax && pot.npr == xa.npr && !ob.pot_radial);
+      if (bare && tabled && keep && doA && !doB && !ob.copy_out && xa.npr == 1) {
+        kept = true;
+        if (epot) form_kept(One{}, std::true_type{}, integral_constant<int, 0>{});
+        else form_kept(One{}, std::false_type{}, integral_constant<int, 0>{});
+      } else if (bare && tabled && epot && !keep && ob.copy_out && shared && xb.ax) {
+        kept = true;
+        if (xa.npr == 1) {
+          if (same) form_kept(One{}, std::true_type{}, One{});
+          else form_kept(One{}, std::true_type{}, Two{});
+        } else {
+          if (same) form_kept(Two{}, std::true_type{}, One{});
+          else form_kept(Two{}, std::true_type{}, Two{});
+        }
+      }
+    }
+    if (kept) {
+    } else if (FEAT == FEAT_X && bare && shared && xb.ax) {
+      if (xa.npr == 1) {
+        if (same) form(integral_constant<int, 1>{}, std::true_type{});
+        else form(integral_constant<int, 1>{}, std::false_type{});
+      } else {
+        if (same) form(integral_constant<int, 2>{}, std::true_type{});
+        else form(integral_constant<int, 2>{}, std::false_type{});
+      }
+    } else if (compact) {
 #pragma unroll
       for (int q = 0; q < SLOTS; ++q) {
         const int ia = PL::xpos(t, q);
@@ -644,13 +766,14 @@ __device__ __forceinline__ void pass_tile(const PassParams& p, const TileGeo<N, 
 // full row passes of 64k threads per line (their line geometry is wave-uniform, in scalar
 // registers; a few spilled
 // bytes cost far less than the fourth wave returns: the 512^3 row pass 2.6 ms at three waves,
-// 1.9 ms at four), three in full column passes; 16-element plans two (full) or three (lean);
+// 1.9 ms at four), three in full column passes and in the boundary tier (its grouped table loads
+// spill 97 registers at four); 16-element plans two (full) or three (lean);
 // the 20- and 24-element plans of the 5*2^k and 3*2^k lengths need their registers and are left
 // uncapped.
 template <int E, int FEAT, bool UNIFORM_LINE>
 constexpr int pass_waves() {
   constexpr bool light = FEAT == FEAT_LEAN || FEAT == FEAT_KIN;
-  if (E <= 8) return (light || UNIFORM_LINE) ? 4 : 3;
+  if (E <= 8) return light || (UNIFORM_LINE && FEAT != FEAT_BOUNDARY) ? 4 : 3;
   if (E <= 16) return light ? 3 : 2;   // (the X tier counts as full)
   return 1;
 }
@@ -702,15 +825,20 @@ __global__ void __launch_bounds__((Geo<Real, N, ROW, V>::THREADS),
   const int64_t k0 = (nb & 7) == 0 ? (int64_t)(blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3) : (int64_t)blockIdx.x;
   TileGeo<N, ROW, W> g;
   g.at(p, tile_at<W, ROW>(p, k0, ntiles), w);
+  // A predicated load whose value is widened at once waits inside its branch (an FP32 state's loads
+  // then come one round trip after another: 320^3 columns 356 us, 263 without the predicate), so idle
+  // lanes read the first line there. The other states keep the predicate: without it the scheduler
+  // mixes these loads with the tables' and the full tier of 2048-point rows goes from 87 to 117 VGPRs.
+  constexpr bool ANY_LANE = S32 || PL::MIXED;
   T v[SLOTS];
   if (PL::MIXED && !(p.flags & F_INV1)) {   // (an inverse alone is an F_INV1: F_INV2 follows F_FWD)
 #pragma unroll
     for (int q = 0; q < SLOTS; ++q)
-      v[q] = g.valid && PL::xhas(t, q) ? from_state<T>(src[g.base + (int64_t)PL::xpos(t, q) * g.step]) : T{Real(0), Real(0)};
+      v[q] = from_state<T>(src[g.base + (int64_t)PL::xpos(t, q) * g.step]);
   } else {
 #pragma unroll
     for (int q = 0; q < E; ++q)
-      v[q] = g.valid ? from_state<T>(src[g.base + (int64_t)(t + TT * q) * g.step]) : T{Real(0), Real(0)};
+      v[q] = ANY_LANE || g.valid ? from_state<T>(src[g.base + (int64_t)(t + TT * q) * g.step]) : T{Real(0), Real(0)};
 #pragma unroll
     for (int q = E; q < SLOTS; ++q) v[q] = T{Real(0), Real(0)};
   }

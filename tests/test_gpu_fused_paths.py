@@ -6,7 +6,7 @@
   tiles, unequal sides, one and two substeps, with and without the kinetic energy, and a stop inside
   a run of steps.
 * CoulombInteraction over both coordinates of a plane with unequal sides (a table factor in FP64).
-* The mixed plan of the 5*2^k lengths at partial tiles.
+* Real-time step boundaries in every form of the row pass, the mixed plan at partial tiles.
 
 Bars as for the axis passes: psi 1e-10 FP64, 1e-4 FP32-mixed, 2e-6 FP32 state; records 1e-9 / 1e-4 /
 1e-5 of each column's largest value (fluxes in FP64 only, where they are a difference of
@@ -134,6 +134,25 @@ def test_coulomb_plane_with_unequal_sides(ctx, shape):
         got, want = both(ctx, shape, T.FP64, pd, f, (4, 1, 3), potential=T.POT_COULOMB, Ncharge=1, Echarge=-1, Nsoft=0.7,
                          absorber=T.ABS_CAP, nCAP=6)
         check(got, want, T.FP64)
+
+
+BOUNDARY_SHAPES = [(80, 80), (160, 160), (64, 64), (80, 80, 80), (64, 64, 64)]
+
+
+@pytest.mark.parametrize("prec", [T.FP64, T.FP32_MIXED, T.FP32_STATE])
+@pytest.mark.parametrize("gauge", [T.GAUGE_VELOCITY, T.GAUGE_LENGTH])
+@pytest.mark.parametrize("shape", BOUNDARY_SHAPES, ids=["x".join(map(str, s)) for s in BOUNDARY_SHAPES])
+def test_real_time_with_and_without_energies(ctx, shape, gauge, prec):
+    """One and two interaction terms along the line, the two halves equal (velocity gauge) or sharing
+    their interaction term (length gauge), the boundary state formed (energies) or not; lengths with
+    eight elements a thread and with the mixed plan."""
+    print(f"[case] boundary {shape} gauge={gauge} prec={prec}", flush=True)
+    f = [T.field_desc([0, T.AXIS_X, T.AXIS_XY, T.AXIS_XYZ][len(shape)], 0.1, 0.3, 2)]
+    for outputs in (T.OUT_NORM | T.OUT_FLUX, T.OUT_NORM | T.OUT_EPOT | T.OUT_EKIN | T.OUT_FLUX):
+        pd = T.prop_desc(T.MODE_RE, 1, 0.04, gauge=gauge, outputs=outputs, borders=[(T.BORDER_BOX, 16)])
+        got, want = both(ctx, shape, prec, pd, f, (3, 1), potential=T.POT_ECKHARDT_SACHA if len(shape) == 3 else T.POT_EBERLY,
+                         Ncharge=2, Echarge=-1, Nsoft=0.5, Esoft=1.0, absorber=T.ABS_CAP, nCAP=8)
+        check(got, want, prec)
 
 
 MIXED_SHAPES = [(80, 20), (20, 80), (160, 48), (24, 320), (320, 12), (640, 40), (1280, 10), (16, 1280), (2560, 8), (8, 2560)]
