@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/qsf_hip.h"
+#include "host_stage.hpp"
 #include "physics.hpp"
 #include "qsf_launch.hpp"
 #include "rows.hpp"
@@ -83,6 +84,7 @@ struct qsf_ctx {
   double* scratch = nullptr;   // this device's address of the no-allocation scratch array
   std::string err;
   hipEvent_t ev[2] = {nullptr, nullptr};
+  qsf::HostStage stage;        // large states on their way to the host
   int marks = 0;
   // live per-kernel timing (qsf_prof_*)
   bool prof = false;
@@ -1018,7 +1020,9 @@ struct Grid {
           }
       srcp = tmp.data();
     }
-    if (prec == QSF_FP64) {
+    if (m * 16 >= HostStage::kLeastBytes) {
+      QSF_HIP(ctx->stage.write(psi.p, srcp, 2 * m, prec != QSF_FP64, st()));
+    } else if (prec == QSF_FP64) {
       QSF_HIP(hipMemcpyAsync(psi.p, srcp, m * 16, hipMemcpyHostToDevice, st()));
     } else {
       aux.ensure(m * 16);
@@ -1033,7 +1037,9 @@ struct Grid {
     QSF_REQUIRE(count == m, QSF_ERR_ARG, "download count must equal the grid size");
     std::vector<double> tmp;
     double* dstp = (rep == QSF_REP_P && isMain && D > 1) ? (tmp.resize(2 * m), tmp.data()) : h;
-    if (prec == QSF_FP64) {
+    if (m * 16 >= HostStage::kLeastBytes) {
+      QSF_HIP(ctx->stage.read(dstp, psi.p, 2 * m, prec != QSF_FP64, st()));
+    } else if (prec == QSF_FP64) {
       QSF_HIP(hipMemcpyAsync(dstp, psi.p, m * 16, hipMemcpyDeviceToHost, st()));
     } else {
       aux.ensure(m * 16);

@@ -6,7 +6,7 @@
   tiles, unequal sides, one and two substeps, with and without the kinetic energy, and a stop inside
   a run of steps.
 * CoulombInteraction over both coordinates of a plane with unequal sides (a table factor in FP64).
-* Real-time step boundaries in every form of the row pass, the mixed plan at partial tiles.
+* Real-time step boundaries in every form of the row pass, the mixed plan, large reads.
 
 Bars as for the axis passes: psi 1e-10 FP64, 1e-4 FP32-mixed, 2e-6 FP32 state; records 1e-9 / 1e-4 /
 1e-5 of each column's largest value (fluxes in FP64 only, where they are a difference of
@@ -167,3 +167,18 @@ def test_mixed_plan_partial_tiles(ctx, shape):
     for prec in (T.FP64, T.FP32_STATE):
         got, want = both(ctx, shape, prec, pd, f, (3, 1), potential=T.POT_COULOMB, Ncharge=1, Echarge=-1, Nsoft=0.7)
         check(got, want, prec)
+
+
+@pytest.mark.parametrize("prec", [T.FP64, T.FP32_MIXED, T.FP32_STATE])
+@pytest.mark.parametrize("shape", [(1024, 1024), (160, 160, 48), (2048, 1280)], ids=["least", "remainder", "ring"])
+def test_large_states_come_whole(ctx, shape, prec):
+    """States read through the pinned slots: whole chunks, a last part of one, more than the ring holds."""
+    from qsf_amd import hip
+    print(f"[case] download {shape} prec={prec}", flush=True)
+    gs = hip.GridSet(ctx, T.grid_desc(len(shape), list(shape), 0.2, precision=prec))
+    rng = np.random.default_rng(3)
+    a = rng.normal(size=gs[0].m) + 1j * rng.normal(size=gs[0].m)
+    gs[0].set_psi(a)
+    want = a if prec == T.FP64 else a.astype(np.complex64).astype(np.complex128)
+    for _ in range(2):
+        assert np.array_equal(gs[0].psi(), want)
